@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -79,6 +80,62 @@ int build_halo(const int* nbr, long long ld, int E, int B, std::vector<int>& hof
     return hmax;
 }
 
+bool build_quad_lists(const int* nbr, long long ld, int E, int B, int hmax, std::vector<int>& list, int& jcap, int& hcap) {
+    const int ntiles = (E + B - 1) / B;
+    std::vector<int> nj(ntiles, 0), nh(ntiles, 0);
+    // one tile's edges and halo entries; false: an edge that is not paired with the edge that
+    // points back (or with itself), which only a form that computes both sides can run
+    auto tile = [&](int t, std::vector<int>& jobs, std::vector<int>& h) {
+        const int lo = t * B, hi = std::min(E, lo + B);
+        jobs.clear();
+        h.clear();
+        for (int k = 0; k < 3; ++k)
+            for (int p = lo; p < hi; ++p) {
+                const int w = nbr[(size_t)k * ld + p];
+                if (w >= 0 && ((w >> 2) < lo || (w >> 2) >= hi)) h.push_back(w);
+            }
+        std::sort(h.begin(), h.end());
+        for (int k = 0; k < 3; ++k)
+            for (int p = lo; p < hi; ++p) {
+                const int w = nbr[(size_t)k * ld + p], row = k * B + p - lo, n = w >> 2;
+                int far = w;  // -tag
+                if (w >= 0 && n >= lo && n < hi) {
+                    if (nbr[(size_t)(w & 3) * ld + n] != ((p << 2) | k)) return false;
+                    far = (w & 3) * B + n - lo;
+                    if (far == row) return false;
+                    if (far < row) continue;  // listed from the other side
+                } else if (w >= 0) {
+                    far = 3 * B + (int)(std::lower_bound(h.begin(), h.end(), w) - h.begin());
+                }
+                jobs.push_back(row | (far + 8) << 9);
+            }
+        return (int)h.size() <= hmax;
+    };
+    std::atomic<bool> ok{true};
+    parallel_for(ntiles, [&](int a, int b) {
+        std::vector<int> jobs, h;
+        for (int t = a; t < b && ok; ++t) {
+            if (!tile(t, jobs, h)) ok = false;
+            nj[t] = (int)jobs.size();
+            nh[t] = (int)h.size();
+        }
+    });
+    if (!ok) return false;
+    jcap = (*std::max_element(nj.begin(), nj.end()) + 15) / 16 * 16;
+    hcap = (*std::max_element(nh.begin(), nh.end()) + 15) / 16 * 16;
+    list.assign((size_t)ntiles * (jcap + hcap), -1);
+    parallel_for(ntiles, [&](int a, int b) {
+        std::vector<int> jobs, h;
+        for (int t = a; t < b; ++t) {
+            tile(t, jobs, h);
+            int* l = &list[(size_t)t * (jcap + hcap)];
+            std::copy(jobs.begin(), jobs.end(), l);
+            std::copy(h.begin(), h.end(), l + jcap);
+        }
+    });
+    return true;
+}
+
 int max_lds_per_block(int device) {
     int v = 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess) return 65536;
@@ -103,6 +160,7 @@ struct rkdg_ctx {
     int* nloc = nullptr;        // staged form: neighbours as LDS slots
     int* hoff = nullptr;        // staged form: per-tile halo offsets
     int* hids = nullptr;        // staged form: halo element positions
+    int quad = 0, jcap = 0, hcap = 0;  // four-lanes-per-element FP64 form and its list capacities
     int lds_stride = 0;         // staged form: doubles per LDS row (block + largest halo)
     int staged = 0;
     int persistent = 0;         // workgroups of the persistent grid (0: one per tile)
@@ -165,6 +223,9 @@ static StageArgs make_args(rkdg_ctx* c, int stage, int slot, int dt_mode, double
     a.hoff = c->hoff;
     a.hids = c->hids;
     a.lds_stride = c->lds_stride;
+    a.quad = c->quad;
+    a.jcap = c->jcap;
+    a.hcap = c->hcap;
     a.staged = c->staged;
     a.persistent = c->persistent;
     a.stagger = c->stagger;
@@ -298,6 +359,12 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     const bool px = bf16 || (prm->precision == RKDG_PREC_FP32_MFMA && env_int("RKDG_PX", 1));
     if (prm->precision != RKDG_PREC_FP64) c->block = px ? px_block(c->P) : 64;
     if (c->block % 64 || c->block < 64 || c->block > 256) { delete c; return fail(nullptr, RKDG_ERR_ARG, "block must be 64..256, multiple of 64"); }
+    // FP64 without a caller block or a switch among the one-lane-per-element forms: four lanes
+    // per element (k_stage_q) at P3, with Roe, and for LF on meshes too small for the
+    // one-lane forms (quad_max_lf).  RKDG_QUAD=0: never, 1: always.
+    const bool want_quad = prm->precision == RKDG_PREC_FP64 && prm->block == 0 && !std::getenv("RKDG_BLOCK") &&
+                           !std::getenv("RKDG_STAGED") && !std::getenv("RKDG_PIPE") && !std::getenv("RKDG_PERSIST") &&
+                           env_int("RKDG_QUAD", c->P == 3 || prm->flux == RKDG_FLUX_ROE || c->E <= quad_max_lf(c->P));
     c->xcd_remap = env_int("RKDG_XCD_REMAP", 1);
     c->ntiles = (c->E + c->block - 1) / c->block;
     c->ld = (long long)((c->E + 255) / 256) * 256;
@@ -436,11 +503,16 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
         }
     }
 
-    // staged form: per-tile halos, used when the tile's LDS image fits
     std::vector<int> hoff, hids, hnloc;
+    if (want_quad && build_quad_lists(hnbr.data(), ld, E, quad_block(c->P), quad_halo(c->P), hids, c->jcap, c->hcap)) {
+        c->quad = 1;
+        c->block = quad_block(c->P);
+        c->ntiles = (c->E + c->block - 1) / c->block;
+    }
+    // staged form: per-tile halos, used when the tile's LDS image fits
     // (measured faster than the global-gather form at P1 and P2)
-    if (px || (prm->precision == RKDG_PREC_FP64 && c->block == staged_block(c->P) &&
-               env_int("RKDG_STAGED", c->P <= 2 ? 1 : 0))) {
+    if (!c->quad && (px || (prm->precision == RKDG_PREC_FP64 && c->block == staged_block(c->P) &&
+               env_int("RKDG_STAGED", c->P <= 2 ? 1 : 0)))) {
         const int hmax = build_halo(hnbr.data(), ld, E, c->block, hoff, hids, hnloc);
         const int stride = px ? px_stride(c->P) : staged_stride(c->P);
         const long long lds = px ? px_lds_bytes(c->P) : (long long)4 * c->Np * stride * (long long)sizeof(double);
@@ -492,6 +564,11 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     CREATECHK(hipMemcpyAsync(c->geo, tgeo.data(), sizeof(double) * tgeo.size(), hipMemcpyHostToDevice, c->stream));
     CREATECHK(hipMemcpyAsync(c->nbr, tnbr.data(), sizeof(int) * tnbr.size(), hipMemcpyHostToDevice, c->stream));
     CREATECHK(hipMemcpyAsync(c->dtflag, hflag.data(), hflag.size(), hipMemcpyHostToDevice, c->stream));
+    if (c->quad) {
+        CREATECHK(hipMalloc(&c->hids, sizeof(int) * hids.size()));
+        c->bytes += sizeof(int) * hids.size();
+        CREATECHK(hipMemcpyAsync(c->hids, hids.data(), sizeof(int) * hids.size(), hipMemcpyHostToDevice, c->stream));
+    }
     if (c->staged) {
         CREATECHK(hipMalloc(&c->nloc, sizeof(int) * hnloc.size()));
         CREATECHK(hipMalloc(&c->hoff, sizeof(int) * hoff.size()));

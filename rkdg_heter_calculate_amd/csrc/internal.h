@@ -141,6 +141,15 @@ void morton_order(int n, const double* bx, const double* by, int32_t* order);
 // Returns the largest halo.
 int build_halo(const int* nbr, long long ld, int E, int B, std::vector<int>& hoff, std::vector<int>& hids,
                std::vector<int>& nloc);
+// Tables of the four-lanes-per-element FP64 form for tiles of B consecutive device positions.
+// Rows of a tile's trace table: edge k of slot s is row k B + s, halo entry h (an out-of-tile
+// neighbour's edge) row 3 B + h.  list holds, per tile, jcap edges and hcap halo entries (-1:
+// none): an edge as row | (far row + 8) << 9 — once for an edge inside the tile, far row = -tag
+// on a boundary — and a halo entry as neighbour position << 2 | its edge, ascending.  jcap and
+// hcap (the largest counts, rounded up to 16) return through the references.  False when the
+// mesh does not admit the form: a tile with more than hmax halo entries, or an in-tile edge
+// whose neighbour's edge does not point back at it.
+bool build_quad_lists(const int* nbr, long long ld, int E, int B, int hmax, std::vector<int>& list, int& jcap, int& hcap);
 int max_lds_per_block(int device);
 
 // Config parser (io.cpp)
@@ -181,6 +190,8 @@ struct StageArgs {
     int lds_stride;        // >= block + largest halo
     int staged;
     int pipe;              // staged form, persistent: next tile's image loaded during the update
+    int quad;              // four-lanes-per-element FP64 form (k_stage_q): hids holds its tile lists
+    int jcap, hcap;        // their capacities per tile (build_quad_lists)
     int stagger;           // persistent grids: the second half of the workgroups starts this
                            // many 8128-cycle sleeps late, so that the two workgroups sharing a
                            // CU alternate their memory and arithmetic phases
@@ -219,6 +230,28 @@ constexpr int px_stride(int P) { return 352; }
 constexpr long long px_lds_bytes(int P) {
     return P <= 2 ? 4LL * ((P + 1) * (P + 2) / 2) * px_stride(P) * 8
                   : 4LL * ((P + 1) * (P + 2) / 2) * px_stride(P) * 4 + 4LL * px_stride(P) * 8;
+}
+
+// Four-lanes-per-element FP64 form (k_stage_q): elements per tile (16 per wave), operand
+// tables, halo capacity and the LDS of a tile.
+constexpr int quad_block(int P) { return P == 3 ? 128 : 64; }
+constexpr int QUAD_OPS = 45;
+constexpr int quad_ops(int P) {
+    const int NG = P == 1 ? 1 : (P == 2 ? 2 : 3), VG = P <= 2 ? 2 : 3;
+    return 3 * VG * NG + 6 * NG;
+}
+// Meshes of at most this many elements run it with LF at P1 and P2 too: the one-lane forms put
+// 256 elements on a workgroup and need one tile per CU at P1 (65,536 elements; P1 LF at 32,768 /
+// 65,522 / 125,000 triangles: 9.4 / 13.3 / 20.4 us per stage against 13.0 / 14.2 / 16.9) and
+// several at P2 (P2 LF at 20,000 / 262,088 / 524,288 / 2.1M: 11.0 / 42.2 / 83.5 / 334 against
+// 16.5 / 45.9 / 86.6 / 308; at 125,000, one exact round of their workgroups, 25.1 against 24.3).
+constexpr int quad_max_lf(int P) { return P == 1 ? 1 << 16 : (P == 2 ? 640000 : 0); }
+// Tile-boundary edges at most (Z-order tiles of 64 have 24-60, of 128 32-76): each of the tile's
+// lanes of a group takes at most one, so never more than the tile's elements.
+constexpr int quad_halo(int P) { return P == 3 ? 80 : 64; }
+constexpr long long quad_lds_bytes(int P) {
+    return 128LL * quad_ops(P) + 32LL * (3 * quad_block(P) + quad_halo(P)) * (P <= 2 ? 3 : 4) +
+           32LL * (quad_block(P) + quad_halo(P)) + 72LL * quad_block(P);
 }
 
 int upload_tables(int P, const DevTables& t);  // per current device

@@ -256,6 +256,10 @@ __device__ __forceinline__ int iter_count(const StageArgs& a) {
 // dt of the current step, identical in every workgroup of the mesh; done = end time reached
 __device__ __forceinline__ double stage_dt(const StageArgs& a, const TileInfo& ti, bool& done) {
     double dt;
+    if (a.dt_mode == DTM_DEVICE && a.stage > 0) {  // as stage 0 fixed it (the end time's clip included)
+        done = a.t_end > 0 && !(a.t_end - ti.st->t[a.slot] > 0);
+        return ti.st->dt[a.slot];
+    }
     if (a.dt_mode == DTM_DEVICE) dt = ti.cfl / __longlong_as_double((long long)ti.st->ws[a.slot]);
     else dt = a.dt_host;
     done = false;
@@ -1113,6 +1117,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGED
     }
 }
 
+#include "stage_q.inc"
 #include "stage_mx.inc"
 #include "stage_px.inc"
 #include "stage_pz.inc"
@@ -1322,7 +1327,12 @@ int launch_stream_copy(const void* src, void* dst, long long bytes, void* stream
 int upload_tables(int P, const DevTables& t) {
     hipError_t rc = hipMemcpyToSymbol(HIP_SYMBOL(c_tab), &t, sizeof(DevTables), (size_t)(P - 1) * sizeof(DevTables),
                                       hipMemcpyHostToDevice);
-    return (int)rc;
+    if (rc != hipSuccess) return (int)rc;
+    double q[QUAD_OPS * 16] = {};
+    if (P == 1) quad_tables<1>(t, q);
+    else if (P == 2) quad_tables<2>(t, q);
+    else quad_tables<3>(t, q);
+    return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_qtab), q, sizeof q, (size_t)(P - 1) * sizeof q, hipMemcpyHostToDevice);
 }
 
 static int grid_blocks(const StageArgs& a) {
@@ -1332,8 +1342,21 @@ static int grid_blocks(const StageArgs& a) {
 }
 
 template <int P, int FLUX>
+static void launch_stage_q(const StageArgs& a, hipStream_t s) {
+    constexpr size_t lds = (size_t)quad_lds_bytes(P);
+    static bool opted = false;  // above 64 KiB the kernel must opt in
+    if (lds > 65536 && !opted)
+        opted = hipFuncSetAttribute((const void*)k_stage_q<P, FLUX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    hipLaunchKernelGGL((k_stage_q<P, FLUX>), dim3(grid_blocks(a)), dim3(Quad<P>::NT), lds, s, a);
+}
+
+template <int P, int FLUX>
 static void launch_stage_pf(int block, const StageArgs& a, hipStream_t s) {
     dim3 grid(grid_blocks(a)), blk(block);
+    if (a.quad) {
+        launch_stage_q<P, FLUX>(a, s);
+        return;
+    }
     if (a.staged) {
         constexpr size_t lds = (size_t)4 * Deg<P>::Np * staged_stride(P) * sizeof(double);
         static bool opted = false;  // above 64 KiB the kernels must opt in

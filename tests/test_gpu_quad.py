@@ -1,0 +1,100 @@
+"""The four-lanes-per-element FP64 form (P3, Roe, and LF on small meshes) at the sizes where its
+tiles can go wrong: partial tiles of 16 elements per wave and 64 or 128 per workgroup, tiles whose
+edges are all boundary or halo edges, and a caller order it must leave to
+the general kernel.  Against the oracle at the FP64 bar (1e-12)."""
+import numpy as np
+import pytest
+
+from rkdg_heter_calculate_amd import BC_FARFIELD, BC_OUTFLOW, BC_REFLECTION, Grid, Solver
+from helpers import make_pair, rel_l2, vortex_grid, vortex_ic
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+# triangles: 4, 32, 62, 64, 66, 126, 130, 522 (wave, tile and layout-tile remainders)
+SIZES = [(2, 1), (4, 4), (31, 1), (8, 4), (11, 3), (9, 7), (5, 13), (9, 29)]
+
+
+def noisy_state(s, seed):
+    """A state near a uniform flow whose traces differ at every point (native basis)."""
+    rng = np.random.default_rng(seed)
+    U = 0.02 * rng.uniform(-1, 1, s.state_shape())
+    U[:, 0] += np.array([1.0, 0.3, 0.2, 2.6])[:, None]
+    return U
+
+
+@pytest.mark.parametrize("P,flux", [(1, "lf"), (1, "roe"), (2, "lf"), (2, "roe"), (3, "lf"), (3, "roe")])
+@pytest.mark.parametrize("bc", [0, BC_FARFIELD, BC_OUTFLOW, BC_REFLECTION])
+def test_tile_remainders(P, flux, bc):
+    for nx, ny in SIZES:
+        if bc == 0 and min(nx, ny) < 3:
+            continue  # not a manifold periodic mesh
+        print(f"case: quad tiles P{P} {flux} bc {bc} {nx}x{ny}", flush=True)
+        g = Grid.splitquad(nx, ny, 0.0, 0.0, 10.0, 10.0 * ny / nx, periodic=bc == 0, diagonal=1, jitter=0.2, seed=nx,
+                           bc=bc or BC_OUTFLOW)
+        fs = [1.0, 0.3, 0.2, 2.6]
+        o, s = make_pair(g, P=P, flux=flux, dt_policy="max", cfl=0.1, freestream=fs)
+        s.set_state(noisy_state(s, nx), basis=1)
+        o.set_state(s.get_state())
+        s.advance(3)
+        o.advance(3)
+        err = rel_l2(s.get_state(), o.get_state(), o.mass())
+        assert np.all(err < TOL), (nx, ny, err)
+        assert np.allclose(s.residual(), o.residual_change(), rtol=1e-9, atol=1e-14)
+        s.close()
+
+
+@pytest.mark.parametrize("P,flux", [(2, "roe"), (3, "lf")])
+def test_against_the_one_lane_form(P, flux, monkeypatch):
+    """The same run with RKDG_QUAD=0: other roundings (the kernels differ), the same scheme."""
+    print(f"case: quad against one-lane P{P} {flux}", flush=True)
+    g = vortex_grid(45, jitter=0.2, diagonal=1, seed=5)
+    kw = dict(degree=P, flux=flux, dt_policy="max", cfl=0.15)
+    s = Solver(g, **kw)
+    monkeypatch.setenv("RKDG_QUAD", "0")
+    r = Solver(g, **kw)
+    U0 = noisy_state(s, 3)
+    for x in (s, r):
+        x.set_state(U0, basis=1)
+        x.advance(10)
+    Us, Ur = s.get_state(basis=1), r.get_state(basis=1)
+    assert not np.array_equal(Us, Ur)
+    assert np.linalg.norm(Us - Ur) < 1e-13 * np.linalg.norm(Ur)
+
+
+@pytest.mark.parametrize("P", [2, 3])
+@pytest.mark.parametrize("nx", [32, 33, 64])
+def test_row_major_orders_at_the_halo_limit(P, nx):
+    """The caller's row-major numbering: a tile of 64 (128) elements is a strip of one or two rows
+    with 64-70 (up to 132) tile-boundary edges, on both sides of what the form holds."""
+    print(f"case: quad halo limit P{P} nx {nx}", flush=True)
+    g = Grid.splitquad(nx, 12, 0.0, 0.0, 10.0, 10.0, periodic=True, diagonal=1, jitter=0.2, seed=3)
+    o, s = make_pair(g, P=P, flux="roe", dt_policy="max", cfl=0.1, order=np.arange(g.n_elements, dtype=np.int32))
+    s.set_state(noisy_state(s, nx), basis=1)
+    o.set_state(s.get_state())
+    s.advance(3)
+    o.advance(3)
+    err = rel_l2(s.get_state(), o.get_state(), o.mass())
+    assert np.all(err < TOL), err
+    s.close()
+
+
+def test_an_order_it_does_not_admit_and_an_end_time():
+    """A random caller order (tiles with more halo edges than the form holds) runs the general
+    kernel; an end time inside the third step clips it."""
+    print("case: quad not admitted, end time", flush=True)
+    g = vortex_grid(20, jitter=0.2, diagonal=1, seed=2)
+    order = np.random.default_rng(0).permutation(g.n_elements).astype(np.int32)
+    o, s = make_pair(g, P=3, flux="roe", dt_policy="max", cfl=0.1, order=order)
+    U0 = vortex_ic(o)
+    s.set_state(U0)
+    s.advance(3)
+    o.advance(3)
+    assert np.all(rel_l2(s.get_state(), o.get_state(), o.mass()) < TOL)
+    s.close()
+    q = Solver(g, degree=3, flux="roe", dt_policy="max", cfl=0.1)
+    q.set_state(U0)
+    dt = q.compute_dt()
+    n, t = q.advance(10, t_end=2.5 * dt)
+    assert n == 3 and abs(t - 2.5 * dt) < 1e-15
+    q.close()
