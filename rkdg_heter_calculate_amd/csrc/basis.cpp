@@ -157,6 +157,15 @@ void build_ref_basis(int P, RefBasis& B) {
         T.recon[0][k] = (a22 * A[k][0] - a12 * A[k][1]) / det;
         T.recon[1][k] = (a11 * A[k][1] - a12 * A[k][0]) / det;
     }
+    // multiplication by xi and eta: psi_j = sum_m C[j][m] mono_m and mono_m = sum_i L[m][i] psi_i
+    for (int j = 0; j < Np; ++j)
+        for (int m = 0; m < Np; ++m)
+            for (int m2 = 0; m2 < Np; ++m2) {
+                if (MX[m2] == MX[m] + 1 && MY[m2] == MY[m])
+                    for (int i = 0; i <= m2; ++i) T.Mxi[i][j] += (double)(B.C[j][m] * L[m2][i]);
+                if (MX[m2] == MX[m] && MY[m2] == MY[m] + 1)
+                    for (int i = 0; i <= m2; ++i) T.Meta[i][j] += (double)(B.C[j][m] * L[m2][i]);
+            }
     // the edge rule applied to a constant flux (same operation order as a rolled accumulation
     // over the points)
     for (int i = 0; i < Np; ++i) {

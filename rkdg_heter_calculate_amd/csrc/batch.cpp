@@ -43,6 +43,8 @@ struct rkdg_batch {
     DevState* st = nullptr;
     double* cfl = nullptr;
     int* tile_mesh = nullptr;
+    int* order_dev = nullptr;   // caller element of each position (state exchange)
+    Transfer xfer;              // pinned chunks of the state transfers
     int ntiles = 0;
     long long steps = 0;
     hipGraphExec_t graph2 = nullptr;
@@ -144,6 +146,21 @@ static int bwavespeed_all(rkdg_batch* b) {
     if (rc) return bfail(b, RKDG_ERR_HIP, hip_error_string(rc));
     b->steps = 0;
     return RKDG_OK;
+}
+
+// One instance's state exchange through the first rows of U[1] (which holds no state between
+// steps: stage 0 writes all of it).
+static ExchangeArgs bexchange(rkdg_batch* b, int i, int32_t basis) {
+    ExchangeArgs x{};
+    x.U = b->U[0];
+    x.rows = b->U[1];
+    x.geo = b->geo;
+    x.order = b->order_dev;
+    x.first = b->off[i];
+    x.n = b->E[i];
+    x.pad = b->E[i];
+    x.basis = basis;
+    return x;
 }
 
 extern "C" {
@@ -337,11 +354,17 @@ int rkdg_batch_create(int32_t n, const rkdg_mesh* meshes, const rkdg_params* par
     BCREATECHK(hipMalloc(&b->dtflag, hflag.size()));
     BCREATECHK(hipMalloc(&b->st, sizeof(DevState) * n));
     BCREATECHK(hipMalloc(&b->cfl, sizeof(double) * n));
+    {
+        std::vector<int> ord(ld, 0);
+        for (int i = 0; i < n; ++i) std::copy(b->order[i].begin(), b->order[i].end(), ord.begin() + b->off[i]);
+        BCREATECHK(hipMalloc(&b->order_dev, sizeof(int) * ld));
+        BCREATECHK(hipMemcpy(b->order_dev, ord.data(), sizeof(int) * ld, hipMemcpyHostToDevice));
+    }
     BCREATECHK(hipMemcpy(b->geo, to_tile_major(hgeo, GEO_ROWS, ld).data(), sizeof(double) * hgeo.size(), hipMemcpyHostToDevice));
     BCREATECHK(hipMemcpy(b->nbr, to_tile_major(hnbr, NBR_ROWS, ld).data(), sizeof(int) * hnbr.size(), hipMemcpyHostToDevice));
     BCREATECHK(hipMemcpy(b->dtflag, hflag.data(), hflag.size(), hipMemcpyHostToDevice));
     BCREATECHK(hipMemcpy(b->cfl, hcfl.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-    b->bytes = 3 * ub + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size();
+    b->bytes = sizeof(int) * (size_t)ld + 3 * ub + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size();
     const bool prec_form = p0.precision != RKDG_PREC_FP64;
     if (b->P <= 2 || prec_form) {
         // staged-form tables for 256-element tiles (instances start on 256-element
@@ -405,6 +428,8 @@ int rkdg_batch_destroy(rkdg_batch* b) {
     if (b->graph2) hipGraphExecDestroy(b->graph2);
     for (int k = 0; k < 3; ++k) hipFree(b->U[k]);
     hipFree(b->geo); hipFree(b->nbr); hipFree(b->dtflag); hipFree(b->st); hipFree(b->cfl); hipFree(b->tile_mesh);
+    hipFree(b->order_dev);
+    transfer_free(b->xfer);
     hipFree(b->nloc); hipFree(b->hoff); hipFree(b->hids);
     if (b->stream) hipStreamDestroy(b->stream);
     delete b;
@@ -417,23 +442,10 @@ int rkdg_batch_set_state(rkdg_batch* b, int32_t i, int32_t basis, const double* 
     const int E = b->E[i], Np = b->Np, P = b->P;
     // the instance's layout tiles are one contiguous block of the tile-major state; its
     // padding columns keep their rest state, so the block is read, updated and written back
-    const size_t blk = (size_t)(E + LAYOUT_TILE - 1) / LAYOUT_TILE * LAYOUT_TILE * 4 * Np;
-    double* dev = b->U[0] + (size_t)b->off[i] * 4 * Np;
-    std::vector<double> h(blk);
-    BCHK(b, hipMemcpyAsync(h.data(), dev, sizeof(double) * blk, hipMemcpyDeviceToHost, b->stream));
-    BCHK(b, hipStreamSynchronize(b->stream));
-    parallel_for(E, [&](int a0, int a1) {
-        double in[4 * MAXNP], o[4 * MAXNP];
-        for (int p = a0; p < a1; ++p) {
-            const int e = b->order[i][p];
-            for (int v = 0; v < 4; ++v)
-                for (int k = 0; k < Np; ++k) in[v * Np + k] = U[((size_t)v * Np + k) * E + e];
-            if (basis == RKDG_BASIS_ELEMENT) element_to_native(P, &b->ex[i][3 * e], &b->ey[i][3 * e], in, o);
-            else std::memcpy(o, in, sizeof(double) * 4 * Np);
-            for (int r = 0; r < 4 * Np; ++r) h[tile_index(r, 4 * Np, p)] = o[r];
-        }
-    });
-    BCHK(b, hipMemcpyAsync(dev, h.data(), sizeof(double) * blk, hipMemcpyHostToDevice, b->stream));
+    // (U[1] holds no state between steps; the instance's padding columns keep their rest state)
+    BCHK(b, (hipError_t)copy_to_device(b->xfer, b->stream, b->U[1], U, sizeof(double) * 4 * Np * (size_t)E));
+    const int xrc = launch_exchange(b->P, bexchange(b, i, basis), false, b->stream);
+    if (xrc) return bfail(b, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(xrc));
     int rc = bwavespeed_all(b);
     if (rc) return rc;
     BCHK(b, hipStreamSynchronize(b->stream));
@@ -443,23 +455,10 @@ int rkdg_batch_set_state(rkdg_batch* b, int32_t i, int32_t basis, const double* 
 int rkdg_batch_get_state(rkdg_batch* b, int32_t i, int32_t basis, double* U) {
     if (!b || i < 0 || i >= b->n || !U) return bfail(b, RKDG_ERR_ARG, "batch_get_state");
     BCHK(b, hipSetDevice(b->dev));
-    const int E = b->E[i], Np = b->Np, P = b->P;
-    const size_t blk = (size_t)(E + LAYOUT_TILE - 1) / LAYOUT_TILE * LAYOUT_TILE * 4 * Np;
-    std::vector<double> h(blk);
-    BCHK(b, hipMemcpyAsync(h.data(), b->U[0] + (size_t)b->off[i] * 4 * Np, sizeof(double) * blk, hipMemcpyDeviceToHost,
-                           b->stream));
-    BCHK(b, hipStreamSynchronize(b->stream));
-    parallel_for(E, [&](int a0, int a1) {
-        double in[4 * MAXNP], o[4 * MAXNP];
-        for (int p = a0; p < a1; ++p) {
-            const int e = b->order[i][p];
-            for (int r = 0; r < 4 * Np; ++r) in[r] = h[tile_index(r, 4 * Np, p)];
-            if (basis == RKDG_BASIS_ELEMENT) native_to_element(P, &b->ex[i][3 * e], &b->ey[i][3 * e], in, o);
-            else std::memcpy(o, in, sizeof(double) * 4 * Np);
-            for (int v = 0; v < 4; ++v)
-                for (int k = 0; k < Np; ++k) U[((size_t)v * Np + k) * E + e] = o[v * Np + k];
-        }
-    });
+    const int E = b->E[i], Np = b->Np;
+    const int xrc = launch_exchange(b->P, bexchange(b, i, basis), true, b->stream);
+    if (xrc) return bfail(b, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(xrc));
+    BCHK(b, (hipError_t)copy_to_host(b->xfer, b->stream, U, b->U[1], sizeof(double) * 4 * Np * (size_t)E));
     return RKDG_OK;
 }
 

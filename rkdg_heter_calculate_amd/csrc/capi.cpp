@@ -26,10 +26,14 @@
 
 namespace rkdg {
 
+int host_threads() {
+    if (const char* s = std::getenv("RKDG_HOST_THREADS")) return std::max(1, std::atoi(s));
+    const unsigned hw = std::thread::hardware_concurrency();
+    return (int)std::min<unsigned>(hw ? hw : 1, 16);
+}
+
 void parallel_for(int n, const std::function<void(int, int)>& body) {
-    unsigned hw = std::thread::hardware_concurrency();
-    int nt = (int)std::min<unsigned>(hw ? hw : 1, 16);
-    if (const char* s = std::getenv("RKDG_HOST_THREADS")) nt = std::max(1, std::atoi(s));
+    const int nt = host_threads();
     if (n < 4096 || nt <= 1) { body(0, n); return; }
     std::vector<std::thread> th;
     int chunk = (n + nt - 1) / nt;
@@ -153,6 +157,8 @@ struct rkdg_ctx {
     int P = 2, Np = 6, Nqv = 7, Nqe = 3, E = 0, block = 256, ntiles = 0, xcd_remap = 1;
     long long ld = 0;
     std::vector<int32_t> order, pos;  // order[p] = caller id at device position p
+    int* order_dev = nullptr;         // the same on the device (state exchange)
+    Transfer xfer;                    // pinned chunks of the state transfers
     std::vector<double> ex, ey;       // [E][3] element vertex coordinates (caller order)
     double* U[3] = {nullptr, nullptr, nullptr};
     double* geo = nullptr;
@@ -551,9 +557,10 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     CREATECHK(hipMalloc(&c->nbr, sizeof(int) * hnbr.size()));
     CREATECHK(hipMalloc(&c->dtflag, hflag.size()));
     CREATECHK(hipMalloc(&c->flags, sizeof(int) * ld));
+    CREATECHK(hipMalloc(&c->order_dev, sizeof(int) * E));
     CREATECHK(hipMalloc(&c->st, sizeof(DevState)));
     CREATECHK(hipMalloc(&c->res_part, sizeof(double) * 2 * c->ntiles));
-    c->bytes = 3 * ubytes + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size() + sizeof(int) * ld +
+    c->bytes = sizeof(int) * (size_t)E + 3 * ubytes + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size() + sizeof(int) * ld +
                sizeof(double) * 2 * c->ntiles;
     for (int b = 0; b < 3; ++b) CREATECHK(hipMemsetAsync(c->U[b], 0, ubytes, c->stream));
     CREATECHK(hipMemsetAsync(c->flags, 0, sizeof(int) * ld, c->stream));
@@ -563,6 +570,7 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     const std::vector<int> tnbr = to_tile_major(hnbr, NBR_ROWS, ld);
     CREATECHK(hipMemcpyAsync(c->geo, tgeo.data(), sizeof(double) * tgeo.size(), hipMemcpyHostToDevice, c->stream));
     CREATECHK(hipMemcpyAsync(c->nbr, tnbr.data(), sizeof(int) * tnbr.size(), hipMemcpyHostToDevice, c->stream));
+    CREATECHK(hipMemcpyAsync(c->order_dev, c->order.data(), sizeof(int) * E, hipMemcpyHostToDevice, c->stream));
     CREATECHK(hipMemcpyAsync(c->dtflag, hflag.data(), hflag.size(), hipMemcpyHostToDevice, c->stream));
     if (c->quad) {
         CREATECHK(hipMalloc(&c->hids, sizeof(int) * hids.size()));
@@ -605,35 +613,40 @@ int rkdg_destroy(rkdg_ctx* c) {
     for (int b = 0; b < 3; ++b) hipFree(c->U[b]);
     hipFree(c->geo); hipFree(c->nbr); hipFree(c->dtflag); hipFree(c->lim); hipFree(c->pairs);
     hipFree(c->nloc); hipFree(c->hoff); hipFree(c->hids);
+    hipFree(c->order_dev);
+    transfer_free(c->xfer);
     hipFree(c->flags); hipFree(c->st); hipFree(c->res_part);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
     return RKDG_OK;
 }
 
+// State exchange: the caller's rows pass through a stage buffer that holds no state (one of
+// U[1], U[2]: only the step-start buffer and, inside a step, the latest stage are live).
+static ExchangeArgs exchange_args(rkdg_ctx* c, double* U, double* rows, int32_t basis) {
+    ExchangeArgs x{};
+    x.U = U;
+    x.rows = rows;
+    x.geo = c->geo;
+    x.order = c->order_dev;
+    x.first = 0;
+    x.n = c->E;
+    x.pad = (int)c->ld;
+    x.basis = basis;
+    return x;
+}
+
 int rkdg_set_state(rkdg_ctx* c, int32_t basis, const double* U) {
     if (!c || !U || (basis != RKDG_BASIS_ELEMENT && basis != RKDG_BASIS_NATIVE)) return fail(c, RKDG_ERR_ARG, "set_state");
     HIPCHK(c, hipSetDevice(c->dev));
-    const int E = c->E, Np = c->Np, P = c->P;
-    const long long ld = c->ld;
-    std::vector<double> h((size_t)4 * Np * ld, 0.0);
-    parallel_for(E, [&](int a, int b) {
-        double in[4 * MAXNP], outv[4 * MAXNP];
-        for (int p = a; p < b; ++p) {
-            int e = c->order[p];
-            for (int v = 0; v < 4; ++v)
-                for (int i = 0; i < Np; ++i) in[v * Np + i] = U[((size_t)v * Np + i) * E + e];
-            if (basis == RKDG_BASIS_ELEMENT) element_to_native(P, &c->ex[3 * e], &c->ey[3 * e], in, outv);
-            else std::memcpy(outv, in, sizeof(double) * 4 * Np);
-            for (int r = 0; r < 4 * Np; ++r) h[tile_index(r, 4 * Np, p)] = outv[r];
-        }
-    });
-    HIPCHK(c, hipMemcpyAsync(c->U[0], h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, (hipError_t)copy_to_device(c->xfer, c->stream, c->U[1], U, sizeof(double) * 4 * c->Np * (size_t)c->E));
+    int rc = launch_exchange(c->P, exchange_args(c, c->U[0], c->U[1], basis), false, c->stream);
+    if (rc) return fail(c, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(rc));
     c->cur = 0;
     c->next_stage = 0;
     c->steps = 0;
     c->have_state = true;
-    int rc = refresh_wavespeed(c, 0, 0.0);
+    rc = refresh_wavespeed(c, 0, 0.0);
     if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return check_physical(c);
@@ -642,22 +655,10 @@ int rkdg_set_state(rkdg_ctx* c, int32_t basis, const double* U) {
 int rkdg_get_state(rkdg_ctx* c, int32_t basis, double* U) {
     if (!c || !U || (basis != RKDG_BASIS_ELEMENT && basis != RKDG_BASIS_NATIVE)) return fail(c, RKDG_ERR_ARG, "get_state");
     HIPCHK(c, hipSetDevice(c->dev));
-    const int E = c->E, Np = c->Np, P = c->P;
-    const long long ld = c->ld;
-    std::vector<double> h((size_t)4 * Np * ld);
-    HIPCHK(c, hipMemcpyAsync(h.data(), c->U[c->cur], sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    parallel_for(E, [&](int a, int b) {
-        double in[4 * MAXNP], outv[4 * MAXNP];
-        for (int p = a; p < b; ++p) {
-            int e = c->order[p];
-            for (int r = 0; r < 4 * Np; ++r) in[r] = h[tile_index(r, 4 * Np, p)];
-            if (basis == RKDG_BASIS_ELEMENT) native_to_element(P, &c->ex[3 * e], &c->ey[3 * e], in, outv);
-            else std::memcpy(outv, in, sizeof(double) * 4 * Np);
-            for (int v = 0; v < 4; ++v)
-                for (int i = 0; i < Np; ++i) U[((size_t)v * Np + i) * E + e] = outv[v * Np + i];
-        }
-    });
+    double* rows = c->U[c->cur == 1 ? 2 : 1];
+    const int rc = launch_exchange(c->P, exchange_args(c, c->U[c->cur], rows, basis), true, c->stream);
+    if (rc) return fail(c, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(rc));
+    HIPCHK(c, (hipError_t)copy_to_host(c->xfer, c->stream, U, rows, sizeof(double) * 4 * c->Np * (size_t)c->E));
     return RKDG_OK;
 }
 
@@ -898,10 +899,10 @@ int rkdg_time(rkdg_ctx* c, double* t, int64_t* steps) {
 int rkdg_get_flags(rkdg_ctx* c, int32_t* flags) {
     if (!c || !flags) return fail(c, RKDG_ERR_ARG, "get_flags");
     HIPCHK(c, hipSetDevice(c->dev));
-    std::vector<int> h(c->ld);
-    HIPCHK(c, hipMemcpyAsync(h.data(), c->flags, sizeof(int) * c->ld, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int p = 0; p < c->E; ++p) flags[c->order[p]] = h[p];
+    int* rows = (int*)c->U[c->cur == 1 ? 2 : 1];  // holds no state (exchange_args)
+    const int rc = launch_flags_out(c->flags, c->order_dev, c->E, rows, c->stream);
+    if (rc) return fail(c, RKDG_ERR_HIP, std::string("flags: ") + hip_error_string(rc));
+    HIPCHK(c, (hipError_t)copy_to_host(c->xfer, c->stream, flags, rows, sizeof(int) * (size_t)c->E));
     return RKDG_OK;
 }
 

@@ -68,6 +68,10 @@ struct DevTables {
     // A (F.xi sum_q w_q d psi_i/d xi + F.eta sum_q w_q d psi_i/d eta) equals
     // sum_k l_k/2 F.n_k Se[k][i], so the precision forms leave both out)
     double Se[3][MAXNP];
+    // multiplication by xi and eta in the basis, up to the degree: (xi f)_i = sum_j Mxi[i][j] f_j
+    // for f of a degree below P (the element basis of the state exchange is built with them)
+    double Mxi[MAXNP][MAXNP];
+    double Meta[MAXNP][MAXNP];
 };
 
 // Device-side step state: wave-speed maxima and times per step parity.
@@ -82,6 +86,19 @@ struct DevState {
 
 // Minimal fork-join helper for host loops (the library carries no OpenMP runtime).
 void parallel_for(int n, const std::function<void(int, int)>& body);
+int host_threads();  // its threads at most (RKDG_HOST_THREADS)
+
+// Pinned chunks for state transfers (transfer.cpp), kept with the context or batch that owns
+// them: at most CHUNKS of 8 MiB, allocated at the first transfer that needs them.
+struct Transfer {
+    static constexpr int CHUNKS = 4;
+    char* pin = nullptr;
+    size_t bytes = 0;
+};
+// Synchronous copies ordered behind the stream's work; return a hipError_t.
+int copy_to_host(Transfer& t, void* stream, void* host, const void* dev, size_t n);
+int copy_to_device(Transfer& t, void* stream, void* dev, const void* host, size_t n);
+void transfer_free(Transfer& t);
 
 // Host-side basis/geometry helpers (basis.cpp)
 struct RefBasis {
@@ -255,6 +272,20 @@ constexpr long long quad_lds_bytes(int P) {
 }
 
 int upload_tables(int P, const DevTables& t);  // per current device
+// State exchange on the device: the tile-major state of n elements from device position first
+// (U: the whole array) <-> caller rows [4 Np][n] in the caller's element order and basis.
+// order[first + i]: the caller element at that position.  On the way in the positions up to pad
+// (at least n) of them are cleared.
+struct ExchangeArgs {
+    double* U;
+    double* rows;
+    const double* geo;
+    const int* order;
+    int first, n, pad;
+    int basis;             // RKDG_BASIS_*
+};
+int launch_exchange(int P, const ExchangeArgs& a, bool out, void* stream);  // out: U -> rows
+int launch_flags_out(const int* flags, const int* order, int n, int* out, void* stream);
 int launch_stage(int P, int flux, int prec, int block, const StageArgs& a, void* stream);
 int launch_wavespeed(int P, const StageArgs& a, int block, void* stream);
 int launch_state_init(DevState* st, int slot, double t, int n, void* stream);

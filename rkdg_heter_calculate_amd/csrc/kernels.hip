@@ -1297,6 +1297,170 @@ __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
     a.flags[e] = flag;
 }
 
+// ---- state exchange ----------------------------------------------------------------------
+// The reference's per-element basis (src/triangleinfo.cpp:433-602) as native coefficients:
+// phi_k = the k-th monomial of X = (x - xc) / sqrt(A), Y = (y - yc) / sqrt(A) made orthogonal to
+// phi_0 .. phi_(k-1).  The native basis is orthonormal, so the element's inner products are dot
+// products of coefficient vectors, and a monomial is its parent times X or Y (linear in xi, eta).
+template <int P>
+struct ExchangeBasis {
+    static constexpr int Np = Deg<P>::Np;
+    static constexpr int dim(int k) { return k == 0 ? 1 : (k < 3 ? 3 : (k < 6 ? 6 : 10)); }  // of degree(phi_k)
+    double phi[Np][Np], inv[Np];  // inv: 1 / (phi_k, phi_k)
+
+    __device__ __forceinline__ void build(const double* geo, int e) {
+        const DevTables& T = c_tab[P - 1];
+        const double area = tmx(geo, 4, GEO_ROWS, e), f = 2.0 * area / sqrt(area);
+        // columns of the Jacobian, scaled: (x1 - x0, y1 - y0) and (x2 - x0, y2 - y0) over sqrt(A)
+        const double x1 = f * tmx(geo, 3, GEO_ROWS, e), x2 = -f * tmx(geo, 1, GEO_ROWS, e);
+        const double y1 = -f * tmx(geo, 2, GEO_ROWS, e), y2 = f * tmx(geo, 0, GEO_ROWS, e);
+        const double x0 = -(x1 + x2) / 3.0, y0 = -(y1 + y2) / 3.0;
+        double m[Np][Np];
+#pragma unroll
+        for (int k = 0; k < Np; ++k) {
+            constexpr int parent[10] = {0, 0, 0, 1, 2, 2, 3, 4, 5, 5};
+            constexpr bool times_y[10] = {false, false, true, false, false, true, false, false, false, true};
+            const int q = parent[k];
+#pragma unroll
+            for (int i = 0; i < Np; ++i) m[k][i] = k == 0 && i == 0 ? 1.0 : 0.0;
+            if (k > 0) {
+                const double a0 = times_y[k] ? y0 : x0, a1 = times_y[k] ? y1 : x1, a2 = times_y[k] ? y2 : x2;
+#pragma unroll
+                for (int i = 0; i < dim(k); ++i) {
+                    double sx = 0.0, sy = 0.0;
+#pragma unroll
+                    for (int j = 0; j < dim(q); ++j) {
+                        sx = fma(T.Mxi[i][j], m[q][j], sx);
+                        sy = fma(T.Meta[i][j], m[q][j], sy);
+                    }
+                    m[k][i] = fma(a1, sx, fma(a2, sy, i < dim(q) ? a0 * m[q][i] : 0.0));
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < Np; ++i) phi[k][i] = m[k][i];
+#pragma unroll
+            for (int l = 0; l < k; ++l) {
+                double ip = 0.0;
+#pragma unroll
+                for (int i = 0; i < dim(l); ++i) ip = fma(m[k][i], phi[l][i], ip);
+                ip *= inv[l];
+#pragma unroll
+                for (int i = 0; i < dim(l); ++i) phi[k][i] = fma(-ip, phi[l][i], phi[k][i]);
+            }
+            double nrm = 0.0;
+#pragma unroll
+            for (int i = 0; i < dim(k); ++i) nrm = fma(phi[k][i], phi[k][i], nrm);
+            inv[k] = 1.0 / nrm;
+        }
+    }
+};
+
+// Tile-major state -> the caller's rows [4 Np][n], one lane per element (a 2.1M-triangle P3 state
+// in the native basis: about 1.5 ms of the 17-30 ms its 671 MB take to the host).
+template <int P, int BASIS>
+__global__ void __launch_bounds__(256) k_state_out(ExchangeArgs a) {
+    constexpr int Np = Deg<P>::Np;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.n) return;
+    const int e = a.first + i, to = a.order[e];
+    double u[4][Np];
+    load_modes<Np>(a.U, e, u);
+    if constexpr (BASIS == RKDG_BASIS_ELEMENT) {
+        ExchangeBasis<P> B;
+        B.build(a.geo, e);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int k = 0; k < Np; ++k) {
+                double s = 0.0;
+#pragma unroll
+                for (int j = 0; j < B.dim(k); ++j) s = fma(u[v][j], B.phi[k][j], s);
+                a.rows[(size_t)(v * Np + k) * a.n + to] = s * B.inv[k];
+            }
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int k = 0; k < Np; ++k) a.rows[(size_t)(v * Np + k) * a.n + to] = u[v][k];
+    }
+}
+
+// The caller's rows -> tile-major state; positions past the elements are cleared.
+template <int P, int BASIS>
+__global__ void __launch_bounds__(256) k_state_in(ExchangeArgs a) {
+    constexpr int Np = Deg<P>::Np;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.pad) return;
+    const int e = a.first + i;
+    double u[4][Np];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int k = 0; k < Np; ++k) u[v][k] = 0.0;
+    if (i < a.n) {
+        const int from = a.order[e];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int k = 0; k < Np; ++k) u[v][k] = a.rows[(size_t)(v * Np + k) * a.n + from];
+        if constexpr (BASIS == RKDG_BASIS_ELEMENT) {
+            ExchangeBasis<P> B;
+            B.build(a.geo, e);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                double d[Np];
+#pragma unroll
+                for (int j = 0; j < Np; ++j) d[j] = 0.0;
+#pragma unroll
+                for (int k = 0; k < Np; ++k)
+#pragma unroll
+                    for (int j = 0; j < B.dim(k); ++j) d[j] = fma(u[v][k], B.phi[k][j], d[j]);
+#pragma unroll
+                for (int j = 0; j < Np; ++j) u[v][j] = d[j];
+            }
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int k = 0; k < Np; ++k) tmx(a.U, v * Np + k, 4 * Np, e) = u[v][k];
+}
+
+template <int P>
+static void launch_exchange_p(const ExchangeArgs& a, bool out, hipStream_t s) {
+    const dim3 grid(((out ? a.n : a.pad) + 255) / 256), blk(256);
+    if (a.basis == RKDG_BASIS_ELEMENT) {
+        if (out) hipLaunchKernelGGL((k_state_out<P, RKDG_BASIS_ELEMENT>), grid, blk, 0, s, a);
+        else hipLaunchKernelGGL((k_state_in<P, RKDG_BASIS_ELEMENT>), grid, blk, 0, s, a);
+    } else {
+        if (out) hipLaunchKernelGGL((k_state_out<P, RKDG_BASIS_NATIVE>), grid, blk, 0, s, a);
+        else hipLaunchKernelGGL((k_state_in<P, RKDG_BASIS_NATIVE>), grid, blk, 0, s, a);
+    }
+}
+
+int launch_exchange(int P, const ExchangeArgs& a, bool out, void* stream) {
+    hipStream_t s = (hipStream_t)stream;
+    switch (P) {
+        case 1: launch_exchange_p<1>(a, out, s); break;
+        case 2: launch_exchange_p<2>(a, out, s); break;
+        case 3: launch_exchange_p<3>(a, out, s); break;
+        default: return (int)hipErrorInvalidValue;
+    }
+    return (int)hipGetLastError();
+}
+
+// Limiter flags in the caller's element order.
+__global__ void __launch_bounds__(256) k_flags_out(const int* __restrict__ flags, const int* __restrict__ order, int n,
+                                                   int* __restrict__ out) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p < n) out[order[p]] = flags[p];
+}
+
+int launch_flags_out(const int* flags, const int* order, int n, int* out, void* stream) {
+    hipLaunchKernelGGL(k_flags_out, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, flags, order, n, out);
+    return (int)hipGetLastError();
+}
+
 // Plain streaming copy (16 bytes per lane per iteration), the calibration kernel for
 // bandwidth and memory counters.
 typedef double dvec2 __attribute__((ext_vector_type(2)));
