@@ -29,6 +29,21 @@
 namespace rkdg {
 
 __constant__ DevTables c_tab[3];
+// Tables that every workgroup copies into its LDS, in the layout it copies: the edge table
+// [edge][point][mode] here, the precision forms' operand tables beside their kernels.  Filling
+// them per workgroup from c_tab cost an index division and a scattered load per entry, about a
+// tenth of a precision form's tile.  upload_tables writes them.
+__device__ double g_ve[3][3 * MAXQE * MAXNP];
+
+// Copies a table of global memory into LDS (size a multiple of 16 bytes, 16-byte aligned).
+template <typename T>
+__device__ __forceinline__ void copy_table(T& lds, const T& src) {
+    static_assert(sizeof(T) % 16 == 0, "copied in 16-byte parts");
+    constexpr int N = sizeof(T) / 16;
+    const uint4* s = reinterpret_cast<const uint4*>(&src);
+    uint4* d = reinterpret_cast<uint4*>(&lds);
+    for (int t = threadIdx.x; t < N; t += blockDim.x) d[t] = s[t];
+}
 
 template <int P>
 struct Deg {
@@ -916,13 +931,9 @@ template <int P, int FLUX>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_stage_pipe(StageArgs a) {
     using L = Staged<P>;
     constexpr int Np = Deg<P>::Np, Nqe = Deg<P>::Nqe;
-    const DevTables& T = c_tab[P - 1];
     __shared__ double sVe[3 * Nqe * Np];
     extern __shared__ __align__(16) double sU[];
-    for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) {
-        const int k = t / (Nqe * Np), r = t - k * (Nqe * Np), j = r / Np, i = r - j * Np;
-        sVe[t] = T.Ve[k][j][i];
-    }
+    for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) sVe[t] = g_ve[P - 1][t];
     const int nit = iter_count(a);
     int it = (int)blockIdx.x - (int)gridDim.x;
     TileInfo ti;
@@ -1008,13 +1019,9 @@ template <int P, int FLUX>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_stage_rp(StageArgs a) {
     using L = Staged<P>;
     constexpr int Np = Deg<P>::Np, Nqe = Deg<P>::Nqe, NR = RpImage<P>::NR, NH = RpImage<P>::NH;
-    const DevTables& T = c_tab[P - 1];
     __shared__ double sVe[3 * Nqe * Np];
     extern __shared__ __align__(16) double sU[];
-    for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) {
-        const int k = t / (Nqe * Np), r = t - k * (Nqe * Np), j = r / Np, i = r - j * Np;
-        sVe[t] = T.Ve[k][j][i];
-    }
+    for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) sVe[t] = g_ve[P - 1][t];
     const int nit = iter_count(a);
     const int G = gridDim.x, tid = threadIdx.x, hh = tid & 127, hr = tid >> 7;
     // tiles of this workgroup's iterations it, it + G, it + 2G, it + 3G (uniform)
@@ -1093,13 +1100,9 @@ template <int P, int FLUX, bool STAGED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGED && P == 1 ? (FLUX == RKDG_FLUX_LF ? 4 : 3) : (STAGED && P <= 2 ? 2 : 1)))) k_stage(StageArgs a) {
     using D = Deg<P>;
     constexpr int Np = D::Np, Nqe = D::Nqe;
-    const DevTables& T = c_tab[P - 1];
     __shared__ double sVe[3 * Nqe * Np];
     extern __shared__ __align__(16) double sU[];
-    for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) {
-        const int k = t / (Nqe * Np), r = t - k * (Nqe * Np), j = r / Np, i = r - j * Np;
-        sVe[t] = T.Ve[k][j][i];
-    }
+    for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) sVe[t] = g_ve[P - 1][t];
     __syncthreads();
     if (a.stagger > 0 && blockIdx.x >= (gridDim.x >> 1))
         for (int i = 0; i < a.stagger; ++i) __builtin_amdgcn_s_sleep(127);
@@ -1488,6 +1491,20 @@ int launch_stream_copy(const void* src, void* dst, long long bytes, void* stream
     return (int)hipGetLastError();
 }
 
+// Fills the tables of degree P that the kernels copy into LDS (one workgroup).
+template <int P>
+__global__ void __launch_bounds__(256) k_fill_tables() {
+    using D = Deg<P>;
+    const DevTables& T = c_tab[P - 1];
+    for (int t = threadIdx.x; t < 3 * D::Nqe * D::Np; t += blockDim.x) {
+        const int k = t / (D::Nqe * D::Np), r = t - k * (D::Nqe * D::Np), j = r / D::Np, i = r - j * D::Np;
+        g_ve[P - 1][t] = T.Ve[k][j][i];
+    }
+    if constexpr (P == 1) fill_px_tab<1>(g_px1, T);
+    else if constexpr (P == 2) fill_px_tab<2>(g_px2, T);
+    else fill_pz_tab<3>(g_pz3, T);
+}
+
 int upload_tables(int P, const DevTables& t) {
     hipError_t rc = hipMemcpyToSymbol(HIP_SYMBOL(c_tab), &t, sizeof(DevTables), (size_t)(P - 1) * sizeof(DevTables),
                                       hipMemcpyHostToDevice);
@@ -1496,7 +1513,13 @@ int upload_tables(int P, const DevTables& t) {
     if (P == 1) quad_tables<1>(t, q);
     else if (P == 2) quad_tables<2>(t, q);
     else quad_tables<3>(t, q);
-    return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_qtab), q, sizeof q, (size_t)(P - 1) * sizeof q, hipMemcpyHostToDevice);
+    rc = hipMemcpyToSymbol(HIP_SYMBOL(g_qtab), q, sizeof q, (size_t)(P - 1) * sizeof q, hipMemcpyHostToDevice);
+    if (rc != hipSuccess) return (int)rc;
+    if (P == 1) hipLaunchKernelGGL(k_fill_tables<1>, dim3(1), dim3(256), 0, nullptr);
+    else if (P == 2) hipLaunchKernelGGL(k_fill_tables<2>, dim3(1), dim3(256), 0, nullptr);
+    else hipLaunchKernelGGL(k_fill_tables<3>, dim3(1), dim3(256), 0, nullptr);
+    rc = hipGetLastError();
+    return (int)(rc == hipSuccess ? hipStreamSynchronize(nullptr) : rc);  // before any other stream reads them
 }
 
 static int grid_blocks(const StageArgs& a) {
