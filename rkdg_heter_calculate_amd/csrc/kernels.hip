@@ -268,22 +268,41 @@ __device__ __forceinline__ int iter_count(const StageArgs& a) {
     return a.xcd_remap ? (a.ntiles + 7) / 8 * 8 : a.ntiles;
 }
 
-// dt of the current step, identical in every workgroup of the mesh; done = end time reached
-__device__ __forceinline__ double stage_dt(const StageArgs& a, const TileInfo& ti, bool& done) {
-    double dt;
-    if (a.dt_mode == DTM_DEVICE && a.stage > 0) {  // as stage 0 fixed it (the end time's clip included)
-        done = a.t_end > 0 && !(a.t_end - ti.st->t[a.slot] > 0);
-        return ti.st->dt[a.slot];
-    }
-    if (a.dt_mode == DTM_DEVICE) dt = ti.cfl / __longlong_as_double((long long)ti.st->ws[a.slot]);
-    else dt = a.dt_host;
+// A value that no workgroup writes during the launch, read at a uniform address through the
+// constant address space: a scalar load, which no wait for vector loads includes.
+template <typename T>
+__device__ __forceinline__ T uniform_load(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)(unsigned long long)p;
+}
+
+// dt of the current step, identical in every workgroup of the mesh, in two parts, so that a
+// kernel can issue the loads with its tile's first ones and wait for them when it needs dt.
+struct StepTime {
+    double x;  // device dt: the wave-speed maximum in stage 0, afterwards the dt stage 0 fixed
+    double t;  // step-start time (with an end time)
+};
+__device__ __forceinline__ StepTime stage_time_load(const StageArgs& a, const TileInfo& ti) {
+    StepTime s{0.0, 0.0};
+    // (stage 0 writes dt[slot] and ws[1 - slot], stage 2 t[1 - slot] and ws[1 - slot])
+    if (a.dt_mode == DTM_DEVICE)
+        s.x = a.stage > 0 ? uniform_load(&ti.st->dt[a.slot]) : __longlong_as_double((long long)uniform_load(&ti.st->ws[a.slot]));
+    if (a.t_end > 0) s.t = uniform_load(&ti.st->t[a.slot]);
+    return s;
+}
+// done = end time reached
+__device__ __forceinline__ double stage_dt(const StageArgs& a, const TileInfo& ti, const StepTime& s, bool& done) {
+    const bool fixed = a.dt_mode == DTM_DEVICE && a.stage > 0;  // (the end time's clip included)
+    double dt = a.dt_mode != DTM_DEVICE ? a.dt_host : (a.stage > 0 ? s.x : ti.cfl / s.x);
     done = false;
     if (a.t_end > 0) {
-        const double rem = a.t_end - ti.st->t[a.slot];
+        const double rem = a.t_end - s.t;
         if (!(rem > 0)) done = true;
-        else if (rem < dt) dt = rem;
+        else if (!fixed && rem < dt) dt = rem;
     }
     return dt;
+}
+__device__ __forceinline__ double stage_dt(const StageArgs& a, const TileInfo& ti, bool& done) {
+    return stage_dt(a, ti, stage_time_load(a, ti), done);
 }
 
 // This tile's pair of residual maxima (stage 2), or NULL when they are not kept.
@@ -711,7 +730,7 @@ template <int P>
 __device__ __forceinline__ int staged_halo_ids(const StageArgs& a, int tile, int (&hid)[Staged<P>::HCH],
                                                int tid = threadIdx.x) {
     const int lane = tid & 63;
-    const int h0 = a.hoff[tile], nh = a.hoff[tile + 1] - h0;
+    const int h0 = uniform_load(a.hoff + tile), nh = uniform_load(a.hoff + tile + 1) - h0;
 #pragma unroll
     for (int hb = 0; hb < Staged<P>::HCH; ++hb) {
         const int h = hb * 32 + (lane >> 1);
@@ -720,10 +739,9 @@ __device__ __forceinline__ int staged_halo_ids(const StageArgs& a, int tile, int
     return nh;
 }
 
-// Issues this wave's share of the direct loads of a tile's image.
+// Issues this wave's share of the direct loads of a tile's image: its own rows, then its halo.
 template <int P>
-__device__ __forceinline__ void staged_fill(const StageArgs& a, int tile, int nh, const int (&hid)[Staged<P>::HCH],
-                                            double* sU, int tid = threadIdx.x) {
+__device__ __forceinline__ void staged_fill_own(const StageArgs& a, int tile, double* sU, int tid = threadIdx.x) {
     using L = Staged<P>;
     const int lane = tid & 63, wave = tid >> 6;
     char* lds = (char*)sU;
@@ -736,6 +754,14 @@ __device__ __forceinline__ void staged_fill(const StageArgs& a, int tile, int nh
         __builtin_amdgcn_global_load_lds((const void*)src,
                                          (__attribute__((address_space(3))) void*)(lds + r * L::S * 8 + part * 1024), 16, 0, 0);
     }
+}
+
+template <int P>
+__device__ __forceinline__ void staged_fill_halo(const StageArgs& a, int nh, const int (&hid)[Staged<P>::HCH], double* sU,
+                                                 int tid = threadIdx.x) {
+    using L = Staged<P>;
+    const int lane = tid & 63, wave = tid >> 6;
+    char* lds = (char*)sU;
 #pragma unroll
     for (int hb = 0; hb < L::HCH; ++hb) {
         if (hb * 32 >= nh) break;  // uniform across the workgroup
@@ -751,38 +777,76 @@ __device__ __forceinline__ void staged_fill(const StageArgs& a, int tile, int nh
     }
 }
 
+// A tile's operands as loaded (the dt flag raw: a test of it would wait for every load in flight).
+struct ElemOpsRaw {
+    int w0, w1, w2;
+    ElemGeo eg;
+    int flag;
+};
+
+// Everything a staged tile reads before its residual, issued so that it costs two round trips to
+// memory: the halo ids, the element's operands, the edge table and the tile's own rows together,
+// then the halo's rows, whose addresses wait for the first.  (A wait for a register load also
+// waits for the direct-to-LDS loads before it, so the register loads come before them.)  One
+// after the other, as the values are used, they were five or six round trips of a tile's 20 us,
+// most of them hidden by the CU's other workgroup: P2 LF at 2.1M triangles 322 -> 317 us per stage,
+// the precision forms at 524,288 BF16 82.3 -> 80.5, FP32 85.5 -> 84.7.  Ends with the tile's barrier.
+template <int P>
+__device__ __forceinline__ ElemOps staged_head(const StageArgs& a, const TileInfo& ti, double* sVe, double* sU, int tid,
+                                               int e, StepTime& step) {
+    constexpr int NVE = 3 * Deg<P>::Nqe * Deg<P>::Np;
+    step = stage_time_load(a, ti);
+    int hid[Staged<P>::HCH];
+    const int nh = staged_halo_ids<P>(a, __builtin_amdgcn_readfirstlane(ti.tile), hid, tid);
+    const int ec = min(e, a.E - 1);  // (lanes past the mesh load its last element's operands and use none)
+    const int w0 = tmx(a.nloc, 0, NBR_ROWS, ec), w1 = tmx(a.nloc, 1, NBR_ROWS, ec), w2 = tmx(a.nloc, 2, NBR_ROWS, ec);
+    const ElemGeo eg{tmx(a.geo, 0, GEO_ROWS, ec), tmx(a.geo, 1, GEO_ROWS, ec), tmx(a.geo, 2, GEO_ROWS, ec),
+                     tmx(a.geo, 3, GEO_ROWS, ec), tmx(a.geo, 4, GEO_ROWS, ec)};
+    const int flag = a.dtflag[a.stage == 2 ? ec : 0];  // (kept raw: a test of it would wait here)
+    double ve = 0.0;
+    if (sVe) ve = g_ve[P - 1][min(tid, NVE - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    staged_fill_own<P>(a, ti.tile, sU, tid);
+    staged_fill_halo<P>(a, nh, hid, sU, tid);
+    if (sVe && tid < NVE) sVe[tid] = ve;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    return ElemOps{w0, w1, w2, eg, a.stage == 2 && flag != 0};
+}
+
 // One workgroup tile, operands loaded from global memory (STAGED: neighbour traces from
 // the tile's LDS image).
 template <int P, int FLUX, bool STAGED>
-__device__ __forceinline__ void stage_tile(const StageArgs& a, const TileInfo& ti, const double* sVe, double* sU,
+__device__ __forceinline__ void stage_tile(const StageArgs& a, const TileInfo& ti, double* sVe, double* sU,
                                            int tid) {
     constexpr int Np = Deg<P>::Np;
-    bool done;
-    const double dt = stage_dt(a, ti, done);
-    stage_bookkeeping(a, ti, dt, done);
-    if (done) return;
-
     const int e = ti.tile * blockDim.x + tid;
     double ws_l = 0.0, r0_l = 0.0, r1_l = 0.0;
     double Uo[4][Np];
     ElemOps o{};
+    double dt;
+    bool done;
     if (STAGED) {
-        int hid[Staged<P>::HCH];
-        const int nh = staged_halo_ids<P>(a, ti.tile, hid, tid);
-        staged_fill<P>(a, ti.tile, nh, hid, sU, tid);
-        if (e < a.E) load_element_ops(a, a.nloc, e, o);  // same round trip as the image
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
+        StepTime step;
+        o = staged_head<P>(a, ti, sVe, sU, tid, e, step);
+        dt = stage_dt(a, ti, step, done);
+        stage_bookkeeping(a, ti, dt, done);
+        if (done) return;
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
             for (int i = 0; i < Np; ++i) Uo[v][i] = sU[(v * Np + i) * Staged<P>::S + tid];
-    } else if (e < a.E) {
+    } else {
+        dt = stage_dt(a, ti, done);
+        stage_bookkeeping(a, ti, dt, done);
+        if (done) return;
+        if (e < a.E) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+            for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int i = 0; i < Np; ++i) Uo[v][i] = tmx(a.U, v * Np + i, 4 * Np, e);
-        load_element_ops(a, a.nbr, e, o);
+                for (int i = 0; i < Np; ++i) Uo[v][i] = tmx(a.U, v * Np + i, 4 * Np, e);
+            load_element_ops(a, a.nbr, e, o);
+        }
     }
 
     if (e < a.E)
@@ -847,14 +911,7 @@ __device__ __forceinline__ void staged_fill_fixed(const StageArgs& a, int tile, 
     }
 }
 
-// The next tile's operands as loaded (the dt flag raw: a test of it here would wait for
-// every load in flight), read at an index clamped into the mesh.
-struct ElemOpsRaw {
-    int w0, w1, w2;
-    ElemGeo eg;
-    int flag;
-};
-
+// The next tile's operands, read at an index clamped into the mesh.
 __device__ __forceinline__ void load_element_ops_clamped(const StageArgs& a, int e, ElemOpsRaw& o) {
     e = min(e, a.E - 1);
     o.w0 = tmx(a.nloc, 0, NBR_ROWS, e);
@@ -1102,8 +1159,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGED
     constexpr int Np = D::Np, Nqe = D::Nqe;
     __shared__ double sVe[3 * Nqe * Np];
     extern __shared__ __align__(16) double sU[];
-    for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) sVe[t] = g_ve[P - 1][t];
-    __syncthreads();
+    if constexpr (!STAGED) {  // (the staged tile loads it with its operands)
+        for (int t = threadIdx.x; t < 3 * Nqe * Np; t += blockDim.x) sVe[t] = g_ve[P - 1][t];
+        __syncthreads();
+    }
     if (a.stagger > 0 && blockIdx.x >= (gridDim.x >> 1))
         for (int i = 0; i < a.stagger; ++i) __builtin_amdgcn_s_sleep(127);
     const int nit = iter_count(a);
