@@ -34,6 +34,10 @@ struct rkdg_batch {
     int* nloc = nullptr;        // staged form tables (P2)
     int* hoff = nullptr;
     int* hids = nullptr;
+    bool quad_ok = false;       // the meshes admit the four-lanes-per-element FP64 tiles
+    int quad = 0;               // ... and the batch runs them
+    int jcap = 0, hcap = 0;     // their list capacities
+    int* qlist = nullptr;       // their tile lists
     bool staged_ok = false;     // the halo of every tile fits the staged LDS image
     int staged = 0;             // staged form in use (chosen by the autotuner)
     double* U[3] = {nullptr, nullptr, nullptr};
@@ -105,7 +109,10 @@ static StageArgs bargs(rkdg_batch* b, int stage, int slot) {
     a.nbr = b->nbr;
     a.nloc = b->nloc;
     a.hoff = b->hoff;
-    a.hids = b->hids;
+    a.hids = b->quad ? b->qlist : b->hids;
+    a.quad = b->quad;
+    a.jcap = b->jcap;
+    a.hcap = b->hcap;
     a.staged = b->staged;
     a.lds_stride = b->prm.precision != RKDG_PREC_FP64 ? px_stride(b->P) : staged_stride(b->P);
     a.dtflag = b->dtflag;
@@ -366,6 +373,15 @@ int rkdg_batch_create(int32_t n, const rkdg_mesh* meshes, const rkdg_params* par
     BCREATECHK(hipMemcpy(b->cfl, hcfl.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     b->bytes = sizeof(int) * (size_t)ld + 3 * ub + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size();
     const bool prec_form = p0.precision != RKDG_PREC_FP64;
+    if (!prec_form && env_int("RKDG_QUAD", 1)) {
+        std::vector<int> list;
+        if (build_quad_lists(hnbr.data(), ld, (int)ld, quad_block(b->P), quad_halo(b->P), list, b->jcap, b->hcap)) {
+            BCREATECHK(hipMalloc(&b->qlist, sizeof(int) * list.size()));
+            BCREATECHK(hipMemcpy(b->qlist, list.data(), sizeof(int) * list.size(), hipMemcpyHostToDevice));
+            b->bytes += sizeof(int) * list.size();
+            b->quad_ok = true;
+        }
+    }
     if (b->P <= 2 || prec_form) {
         // staged-form tables for 256-element tiles (instances start on 256-element
         // boundaries, so no tile spans two instances): the FP64 form's at P1/P2, the
@@ -398,8 +414,7 @@ int rkdg_batch_create(int32_t n, const rkdg_mesh* meshes, const rkdg_params* par
         b->block = px_block(b->P);
         b->staged = 1;
     }
-    // FP64: the global-gather tiles until rkdg_batch_autotune picks; RKDG_BATCH_STAGED=1
-    // starts from the staged tiles instead (when every halo fits)
+    // FP64: RKDG_BATCH_STAGED=1 starts from the staged tiles (when every halo fits)
     if (p0.precision == RKDG_PREC_FP64 && b->staged_ok && env_int("RKDG_BATCH_STAGED", 0)) {
         b->block = staged_block(b->P);
         b->staged = 1;
@@ -408,6 +423,22 @@ int rkdg_batch_create(int32_t n, const rkdg_mesh* meshes, const rkdg_params* par
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, b->dev) == hipSuccess && prop.multiProcessorCount > 0) cus = prop.multiProcessorCount;
     b->persistent = cus * 8;
+    // without a caller block: the form a single mesh of the batch's size would run (rkdg_create).
+    // 48 meshes of 32-192 quads a side (1.0M triangles), ms per step, global-gather tiles (the
+    // general form) / staged / four lanes per element: P2 LF 0.70 / 0.48 / 0.50, P2 Roe
+    // 0.82 / 0.63 / 0.53, P1 LF 0.33 / 0.29 / 0.35, P1 Roe 0.41 / 0.39 / 0.38, P3 LF
+    // 1.17 / - / 0.76; 48 of 32-64 (197,000), P2 LF 0.180 / 0.131 / 0.113
+    if (!prec_form && p0.block == 0 && !b->staged) {
+        if (b->quad_ok && (b->P == 3 || p0.flux == RKDG_FLUX_ROE || b->ld <= quad_max_lf(b->P))) {
+            b->quad = 1;
+            b->block = quad_block(b->P);
+            b->persistent = 0;
+        } else if (b->staged_ok) {
+            b->staged = 1;
+            b->block = staged_block(b->P);
+            b->persistent = 0;
+        }
+    }
     int rc = upload_tables(b->P, ref_basis(b->P).tab);
     if (rc) { rkdg_batch_destroy(b); return bfail(nullptr, RKDG_ERR_HIP, "table upload"); }
     rc = upload_tiles(b);
@@ -430,6 +461,7 @@ int rkdg_batch_destroy(rkdg_batch* b) {
     hipFree(b->geo); hipFree(b->nbr); hipFree(b->dtflag); hipFree(b->st); hipFree(b->cfl); hipFree(b->tile_mesh);
     hipFree(b->order_dev);
     transfer_free(b->xfer);
+    hipFree(b->qlist);
     hipFree(b->nloc); hipFree(b->hoff); hipFree(b->hids);
     if (b->stream) hipStreamDestroy(b->stream);
     delete b;
@@ -571,8 +603,10 @@ static bool tiles_valid(const rkdg_batch* b, int staged, int block, int per_cu) 
     return block == 64 || block == 128 || block == 256;
 }
 
+// staged: 0, 1, or 2 for the four-lanes-per-element tiles (block quad_block, per_cu 0)
 static int apply_tiles(rkdg_batch* b, int staged, int block, int per_cu) {
-    b->staged = staged;
+    b->staged = staged == 1;
+    b->quad = staged == 2;
     b->block = block;
     b->persistent = per_cu ? device_cus(b->dev) * per_cu * 256 / block : 0;
     return upload_tiles(b);
@@ -591,7 +625,7 @@ int rkdg_batch_set_tiles(rkdg_batch* b, int32_t staged, int32_t block, int32_t p
 int rkdg_batch_get_tiles(rkdg_batch* b, int32_t out[3]) {
     if (!b || !out) return bfail(b, RKDG_ERR_ARG, "batch_get_tiles");
     const int cus = device_cus(b->dev);
-    out[0] = b->staged;
+    out[0] = b->quad ? 2 : b->staged;
     out[1] = b->block;
     out[2] = b->persistent ? b->persistent * b->block / (256 * cus) : 0;
     return RKDG_OK;
@@ -603,7 +637,7 @@ int rkdg_batch_autotune(rkdg_batch* b, int32_t* best_block) {
     const int cands[3] = {64, 128, 256};
     const int pers[3] = {0, 4, 8};  // 0: one workgroup per tile; else workgroups per CU
     float best = 1e30f;
-    int bb = b->block, bs = b->staged;
+    int bb = b->block, bs = b->quad ? 2 : b->staged;
     int bp = 0;
     {
         int32_t cur[3];
@@ -618,10 +652,10 @@ int rkdg_batch_autotune(rkdg_batch* b, int32_t* best_block) {
         hipEventDestroy(e1);
         return bfail(b, code, m);
     };
-    for (int st = 0; st <= 1; ++st)
+    for (int st = 0; st <= 2; ++st)
         for (int c : cands)
             for (int pw : pers) {
-                if (!tiles_valid(b, st, c, pw)) continue;
+                if (st < 2 ? !tiles_valid(b, st, c, pw) : !(b->quad_ok && c == quad_block(b->P) && pw == 0)) continue;
                 int rc = apply_tiles(b, st, c, pw);
                 if (rc) return finish(rc, b->err);
                 // stage 1 reads buffers 1 and 0 and writes buffer 2: repeatable without

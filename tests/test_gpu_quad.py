@@ -5,7 +5,7 @@ the general kernel.  Against the oracle at the FP64 bar (1e-12)."""
 import numpy as np
 import pytest
 
-from rkdg_heter_calculate_amd import BC_FARFIELD, BC_OUTFLOW, BC_REFLECTION, Grid, Solver
+from rkdg_heter_calculate_amd import BASIS_NATIVE, BC_FARFIELD, BC_OUTFLOW, BC_REFLECTION, Batch, Grid, Solver
 from helpers import make_pair, rel_l2, vortex_grid, vortex_ic
 
 pytestmark = pytest.mark.gpu
@@ -98,3 +98,30 @@ def test_an_order_it_does_not_admit_and_an_end_time():
     n, t = q.advance(10, t_end=2.5 * dt)
     assert n == 3 and abs(t - 2.5 * dt) < 1e-15
     q.close()
+
+
+@pytest.mark.parametrize("P,flux", [(1, "roe"), (2, "lf"), (2, "roe"), (3, "lf")])
+def test_batch_instances_equal_single_meshes(P, flux):
+    """A batch without a caller block runs the same tiles as a single mesh (instances start on
+    256-element boundaries, so their tiles hold the same elements): the same bits.  24, 130 and 512
+    triangles: a partial tile, a partial layout tile and two full ones."""
+    print(f"case: quad batch P{P} {flux}", flush=True)
+    grids = [Grid.splitquad(nx, ny, 0.0, 0.0, 10.0, 10.0, periodic=True, diagonal=1, jitter=0.2, seed=nx)
+             for nx, ny in ((4, 3), (5, 13), (16, 16))]
+    kw = dict(degree=P, flux=flux, dt_policy="max", cfl=0.1)
+    b = Batch(grids, [kw] * 3)
+    assert b.tiles()["staged"] == 2
+    singles = [Solver(g, **kw) for g in grids]
+    for i, s in enumerate(singles):
+        U = noisy_state(s, i)
+        b.set_state(i, U, BASIS_NATIVE)
+        s.set_state(U, BASIS_NATIVE)
+    b.advance(5)
+    b.sync()
+    for i, s in enumerate(singles):
+        s.advance(5)
+        assert np.array_equal(b.get_state(i, BASIS_NATIVE), s.get_state(BASIS_NATIVE)), i
+        assert b.time(i) == s.time()[0]
+    with pytest.raises(Exception):  # chosen by the library, not through set_tiles
+        b.set_tiles(2, b.tiles()["block"], 0)
+    b.close()
