@@ -142,6 +142,11 @@ void build_ref_basis(int P, RefBasis& B) {
     for (int q = 0; q < nq; ++q) T.Vv[q][0] = 1.0;
     for (int k = 0; k < 3; ++k)
         for (int j = 0; j < ne; ++j) T.Ve[k][j][0] = 1.0;
+    for (int i = 0; i < Np; ++i) {
+        for (int q = 0; q < nq; ++q) T.pmax[i] = std::max(T.pmax[i], std::fabs(T.Vv[q][i]));
+        for (int k = 0; k < 3; ++k)
+            for (int j = 0; j < ne; ++j) T.pmax[i] = std::max(T.pmax[i], std::fabs(T.Ve[k][j][i]));
+    }
     // limiter: P1 modes at the edge midpoints and the least-squares slope recovery
     double A[3][2];
     for (int k = 0; k < 3; ++k) {

@@ -63,6 +63,7 @@ struct DevTables {
     double minv[MAXNP];            // 1 / (quadrature mass per unit area)
     double Vmid[3][3];             // P1 modes at the edge midpoints (limiter)
     double recon[2][3];            // modes 1,2 from midpoint deviations (limiter)
+    double pmax[MAXNP];            // largest |psi_i| at the volume and edge points (limiter)
     // the edge rule applied to a constant flux, sum_j we_j psi_i(edge k point j): the BF16
     // precision forms' edge corrections (for a constant flux the volume rule's
     // A (F.xi sum_q w_q d psi_i/d xi + F.eta sum_q w_q d psi_i/d eta) equals

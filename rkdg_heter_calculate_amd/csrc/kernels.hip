@@ -1241,6 +1241,13 @@ __global__ void k_state_init(DevState* st, int n, int slot, double t) {
 // race-free.  Flags: bit 0 TVB-limited, bit 1 positivity-scaled.
 constexpr double POS_EPS = 1e-13;
 
+//
+// Bound: the bytes of the state it reads.  Most elements of a flow need neither half of it, so
+// each is entered only by elements that may: a component whose midpoint deviations are all
+// within M h^2 keeps them whatever the neighbours are, so an element without a larger one reads no
+// neighbours and no limiter geometry (60 of 172 bytes at P1); and a bound on density and
+// pressure over all points at once (sums of |mode| times the largest |psi|) rules the
+// positivity loop (16 points and divisions at P1) out.
 template <int P>
 __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
     using D = Deg<P>;
@@ -1249,106 +1256,129 @@ __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= a.E) return;
     if (a.t_end > 0 && !(a.t_end - a.st->t[a.slot] > 0)) return;  // past the end time (as its stage)
-    double c[4][Np], nm[3][4];
+    double c[4][Np];
 #pragma unroll
     for (int v = 0; v < 4; ++v)
 #pragma unroll
         for (int i = 0; i < Np; ++i) c[v][i] = tmx(a.U, v * Np + i, 4 * Np, e);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const int w = tmx(a.nbr, k, NBR_ROWS, e);
-        if (w >= 0) {
-            const int n = w >> 2;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) nm[k][v] = tmx(a.U, v * Np, 4 * Np, n);
-        } else {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) nm[k][v] = c[v][0];
-        }
-    }
-    double al[6];
-#pragma unroll
-    for (int r = 0; r < 6; ++r) al[r] = tmx(a.lim, r, LIM_ROWS, e);
     const double tol = a.M * tmx(a.lim, 6, LIM_ROWS, e);
-    const int pk = a.pairs[e];
+    bool beyond = false;  // a midpoint deviation beyond M h^2 (or NaN)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) beyond |= !(fabs(T.Vmid[k][1] * c[v][1] + T.Vmid[k][2] * c[v][2]) <= tol);
     const double nu = 1.5;
     int flag = 0;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const double m0 = c[v][0];
-        double d[3];
-        bool changed = false;
+    if (beyond) {
+        double nm[3][4], al[6];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const double ut = T.Vmid[k][1] * c[v][1] + T.Vmid[k][2] * c[v][2];
-            const int k1 = (pk >> (4 * k)) & 3, k2 = (pk >> (4 * k + 2)) & 3;
-            double n1 = nm[0][v], n2 = nm[0][v];
-            if (k1 == 1) n1 = nm[1][v]; else if (k1 == 2) n1 = nm[2][v];
-            if (k2 == 1) n2 = nm[1][v]; else if (k2 == 2) n2 = nm[2][v];
-            const double b = nu * (al[2 * k] * (n1 - m0) + al[2 * k + 1] * (n2 - m0));
-            double r;
-            if (fabs(ut) <= tol) r = ut;
-            else if (ut > 0 && b > 0) r = fmin(ut, b);
-            else if (ut < 0 && b < 0) r = fmax(ut, b);
-            else r = 0.0;
-            if (r != ut) changed = true;
-            d[k] = r;
+            const int w = tmx(a.nbr, k, NBR_ROWS, e);
+            if (w >= 0) {
+                const int n = w >> 2;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) nm[k][v] = tmx(a.U, v * Np, 4 * Np, n);
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) nm[k][v] = c[v][0];
+            }
         }
-        if (!changed) continue;
-        flag = 1;
-        const double sum = d[0] + d[1] + d[2];
-        if (sum != 0.0) {
-            double pos = 0, neg = 0;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) { pos += fmax(0.0, d[k]); neg += fmax(0.0, -d[k]); }
-            const double tp = pos > 0 ? fmin(1.0, neg / pos) : 0.0;
-            const double tn = neg > 0 ? fmin(1.0, pos / neg) : 0.0;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) d[k] = tp * fmax(0.0, d[k]) - tn * fmax(0.0, -d[k]);
-        }
-        c[v][1] = T.recon[0][0] * d[0] + T.recon[0][1] * d[1] + T.recon[0][2] * d[2];
-        c[v][2] = T.recon[1][0] * d[0] + T.recon[1][1] * d[1] + T.recon[1][2] * d[2];
-#pragma unroll
-        for (int i = 3; i < Np; ++i) c[v][i] = 0.0;
-    }
-    // positivity: density first, then pressure, at every volume and edge point
-    const double g = a.gamma;
-    const double rm = c[0][0];
-    double rmin = rm;
-#pragma unroll
-    for (int q = 0; q < Nqv + 3 * Nqe; ++q) {
-        double s = c[0][0];
-#pragma unroll
-        for (int i = 1; i < Np; ++i) s += (q < Nqv ? T.Vv[q][i] : T.Ve[(q - Nqv) / Nqe][(q - Nqv) % Nqe][i]) * c[0][i];
-        rmin = fmin(rmin, s);
-    }
-    double th1 = 1.0;
-    if (rmin < POS_EPS) th1 = fmin(1.0, (rm - POS_EPS) / (rm - rmin));
-    if (th1 < 1.0) {
-#pragma unroll
-        for (int i = 1; i < Np; ++i) c[0][i] *= th1;
-    }
-    const double pm = (g - 1.0) * (c[3][0] - 0.5 * (c[1][0] * c[1][0] + c[2][0] * c[2][0]) / rm);
-    double th2 = 1.0;
-#pragma unroll
-    for (int q = 0; q < Nqv + 3 * Nqe; ++q) {
-        double U[4];
+        for (int r = 0; r < 6; ++r) al[r] = tmx(a.lim, r, LIM_ROWS, e);
+        const int pk = a.pairs[e];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            double s = c[v][0];
+            const double m0 = c[v][0];
+            double d[3];
+            bool changed = false;
 #pragma unroll
-            for (int i = 1; i < Np; ++i) s += (q < Nqv ? T.Vv[q][i] : T.Ve[(q - Nqv) / Nqe][(q - Nqv) % Nqe][i]) * c[v][i];
-            U[v] = s;
+            for (int k = 0; k < 3; ++k) {
+                const double ut = T.Vmid[k][1] * c[v][1] + T.Vmid[k][2] * c[v][2];
+                const int k1 = (pk >> (4 * k)) & 3, k2 = (pk >> (4 * k + 2)) & 3;
+                double n1 = nm[0][v], n2 = nm[0][v];
+                if (k1 == 1) n1 = nm[1][v]; else if (k1 == 2) n1 = nm[2][v];
+                if (k2 == 1) n2 = nm[1][v]; else if (k2 == 2) n2 = nm[2][v];
+                const double b = nu * (al[2 * k] * (n1 - m0) + al[2 * k + 1] * (n2 - m0));
+                double r;
+                if (fabs(ut) <= tol) r = ut;
+                else if (ut > 0 && b > 0) r = fmin(ut, b);
+                else if (ut < 0 && b < 0) r = fmax(ut, b);
+                else r = 0.0;
+                if (r != ut) changed = true;
+                d[k] = r;
+            }
+            if (!changed) continue;
+            flag = 1;
+            const double sum = d[0] + d[1] + d[2];
+            if (sum != 0.0) {
+                double pos = 0, neg = 0;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) { pos += fmax(0.0, d[k]); neg += fmax(0.0, -d[k]); }
+                const double tp = pos > 0 ? fmin(1.0, neg / pos) : 0.0;
+                const double tn = neg > 0 ? fmin(1.0, pos / neg) : 0.0;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) d[k] = tp * fmax(0.0, d[k]) - tn * fmax(0.0, -d[k]);
+            }
+            c[v][1] = T.recon[0][0] * d[0] + T.recon[0][1] * d[1] + T.recon[0][2] * d[2];
+            c[v][2] = T.recon[1][0] * d[0] + T.recon[1][1] * d[1] + T.recon[1][2] * d[2];
+#pragma unroll
+            for (int i = 3; i < Np; ++i) c[v][i] = 0.0;
         }
-        const double pq = (g - 1.0) * (U[3] - 0.5 * (U[1] * U[1] + U[2] * U[2]) / U[0]);
-        if (pq < POS_EPS) th2 = fmin(th2, (pm - POS_EPS) / (pm - pq));
     }
-    if (th1 < 1.0 || th2 < 1.0) {
-        flag |= 2;
+    // bounds over all points: rho >= rlo, |m| <= mhi, rho E >= elo, hence p >= plo.  Beyond the
+    // margin (rounding is 1e-15 of the mean) no point is below POS_EPS and nothing is scaled.
+    const double g = a.gamma;
+    bool scale;
+    {
+        double dev[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int i = 1; i < Np; ++i) c[v][i] *= th2;
+            for (int i = 1; i < Np; ++i) dev[v] = fma(fabs(c[v][i]), T.pmax[i], dev[v]);
+        const double rlo = c[0][0] - dev[0], elo = c[3][0] - dev[3];
+        const double m1 = fabs(c[1][0]) + dev[1], m2 = fabs(c[2][0]) + dev[2];
+        const double plo = (g - 1.0) * (elo - 0.5 * (m1 * m1 + m2 * m2) * frcp(rlo));
+        scale = !(rlo > fmax(1e-10 * c[0][0], 2 * POS_EPS) && plo > fmax(1e-10 * c[3][0], 2 * POS_EPS));
+    }
+    if (scale) {
+        // positivity: density first, then pressure, at every volume and edge point
+        const double rm = c[0][0];
+        double rmin = rm;
+#pragma unroll
+        for (int q = 0; q < Nqv + 3 * Nqe; ++q) {
+            double s = c[0][0];
+#pragma unroll
+            for (int i = 1; i < Np; ++i) s += (q < Nqv ? T.Vv[q][i] : T.Ve[(q - Nqv) / Nqe][(q - Nqv) % Nqe][i]) * c[0][i];
+            rmin = fmin(rmin, s);
+        }
+        double th1 = 1.0;
+        if (rmin < POS_EPS) th1 = fmin(1.0, (rm - POS_EPS) / (rm - rmin));
+        if (th1 < 1.0) {
+#pragma unroll
+            for (int i = 1; i < Np; ++i) c[0][i] *= th1;
+        }
+        const double pm = (g - 1.0) * (c[3][0] - 0.5 * (c[1][0] * c[1][0] + c[2][0] * c[2][0]) / rm);
+        double th2 = 1.0;
+#pragma unroll
+        for (int q = 0; q < Nqv + 3 * Nqe; ++q) {
+            double U[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                double s = c[v][0];
+#pragma unroll
+                for (int i = 1; i < Np; ++i) s += (q < Nqv ? T.Vv[q][i] : T.Ve[(q - Nqv) / Nqe][(q - Nqv) % Nqe][i]) * c[v][i];
+                U[v] = s;
+            }
+            const double pq = (g - 1.0) * (U[3] - 0.5 * (U[1] * U[1] + U[2] * U[2]) / U[0]);
+            if (pq < POS_EPS) th2 = fmin(th2, (pm - POS_EPS) / (pm - pq));
+        }
+        if (th1 < 1.0 || th2 < 1.0) {
+            flag |= 2;
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int i = 1; i < Np; ++i) c[v][i] *= th2;
+        }
     }
     if (flag) {
 #pragma unroll

@@ -586,3 +586,34 @@ def test_tiles_whose_halo_does_not_fit_the_staged_image():
     f.close()
     with pytest.raises(Exception, match="halo does not fit"):
         Solver(g, order=order, degree=2, flux="lf", dt_policy="max", cfl=0.3, precision="bf16")
+
+
+@pytest.mark.parametrize("P", [1, 2, 3])
+def test_limiter_branches_match_oracle(P):
+    """One stage of dt = 0 (LF, whose wave speed takes cell means only) applies the limiter to the
+    start state: cells within M h^2, beyond it, near vacuum and with negative pressures at points,
+    so that every combination of its two halves is entered and left out, flags included."""
+    print(f"case: limiter branches P{P}", flush=True)
+    g = Grid.splitquad(24, 19, 0.0, 0.0, 1.0, 1.0, periodic=False, diagonal=1, jitter=0.2, seed=9)
+    o, s = make_pair(g, P=P, flux="lf", limiter=True, dt_policy="max", cfl=0.1, tvb_M=50.0)
+    rng = np.random.default_rng(P)
+    E = g.n_elements
+    U = rng.uniform(-1, 1, s.state_shape())
+    U *= (10.0 ** rng.uniform(-6, -0.5, E))[None, None, :]   # deviations from tiny to a third of the mean
+    rho = 10.0 ** rng.uniform(-2, 0, E)
+    p = 10.0 ** rng.uniform(-5, 2, E)
+    U *= rho[None, None, :]
+    U[0, 0], U[1, 0], U[2, 0] = rho, 0.3 * rho, -0.2 * rho
+    U[3, 0] = p / 0.4 + 0.5 * rho * 0.13
+    U[:3, 1:, :E // 3] = 0.0  # a third with smooth density and momentum: limited in rho E, not scaled
+    U[3, 1:, :E // 3] = 0.02 * U[3, 0, :E // 3] * rng.uniform(-1, 1, U[3, 1:, :E // 3].shape)
+    s.set_state(U, basis=1)
+    o.set_state(s.get_state())
+    s.stage(0, 0.0)
+    o.stage(0, 0.0)
+    fs, fo = s.flags(), o.flags()
+    assert set(np.unique(fo)) == {0, 1, 2, 3}
+    assert np.array_equal(fs, fo)
+    err = rel_l2(s.get_state(), o.get_state(), o.mass())
+    assert np.all(err < TOL), err
+    s.close()
