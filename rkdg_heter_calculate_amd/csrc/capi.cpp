@@ -359,8 +359,8 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     c->E = m->n_elements;
     // P3: 64-element tiles (measured 3.5% faster than 128 and 10% faster than 256 at 2.1M)
     c->block = prm->block > 0 ? prm->block : env_int("RKDG_BLOCK", prm->degree >= 3 ? 64 : 256);
-    // precision form: staged tiles of 256 elements (lane per element), else 64 elements on
-    // 256 threads (four lanes per element)
+    // precision form: staged tiles of 256 elements (lane per element; at P3, below, four lanes per
+    // element on 128), else 64 elements on 256 threads (four lanes per element)
     const bool bf16 = prm->precision == RKDG_PREC_BF16_MFMA;
     const bool px = bf16 || (prm->precision == RKDG_PREC_FP32_MFMA && env_int("RKDG_PX", 1));
     if (prm->precision != RKDG_PREC_FP64) c->block = px ? px_block(c->P) : 64;
@@ -536,7 +536,16 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
             c->stagger = env_int("RKDG_STAGGER", 0);
         }
     }
-    if (px && !c->staged) {
+    // P3 precision forms: four lanes per element (k_stage_qf) on a mesh that the staged tiles admit
+    // too (what they refuse stays refused), up to the tiles the allocation-free step accepts
+    if (px && c->staged && c->P == 3 && prm->block == 0 && (c->E - 1) / quad_block(3) < NOALLOC_MAX_TILES && env_int("RKDG_QUAD", 1) && !std::getenv("RKDG_PERSIST") &&
+        build_quad_lists(hnbr.data(), ld, E, quad_block(3), quad_halo(3), hids, c->jcap, c->hcap)) {
+        c->quad = 1;
+        c->staged = c->pipe = c->persistent = 0;
+        c->block = quad_block(3);
+        c->ntiles = (c->E + c->block - 1) / c->block;
+    }
+    if (px && !c->staged && !c->quad) {
         if (bf16) {  // the BF16 contractions run on the staged tiles only
             delete c;
             return fail(nullptr, RKDG_ERR_ARG, "RKDG_PREC_BF16_MFMA: a tile's halo does not fit the staged LDS image");

@@ -1183,6 +1183,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGED
 #include "stage_mx.inc"
 #include "stage_px.inc"
 #include "stage_pz.inc"
+#include "stage_qf.inc"
 
 // CFL wave speed of the current state, max-reduced into ws[slot]
 template <int P>
@@ -1591,7 +1592,10 @@ __global__ void __launch_bounds__(256) k_fill_tables() {
     }
     if constexpr (P == 1) fill_px_tab<1>(g_px1, T);
     else if constexpr (P == 2) fill_px_tab<2>(g_px2, T);
-    else fill_pz_tab<3>(g_pz3, T);
+    else {
+        fill_pz_tab<3>(g_pz3, T);
+        fill_qf_tab(g_qf, T);
+    }
 }
 
 int upload_tables(int P, const DevTables& t) {
@@ -1681,6 +1685,14 @@ static void launch_stage_px_p(int flux, const StageArgs& a, hipStream_t s) {
 
 template <int FLUX, int CT>
 static void launch_stage_pz_f(const StageArgs& a, hipStream_t s) {
+    if (a.quad) {
+        constexpr size_t lds = qf_lds(FLUX, CT);
+        static bool opted_q = false;  // above 64 KiB the kernel must opt in
+        if (lds > 65536 && !opted_q)
+            opted_q = hipFuncSetAttribute((const void*)k_stage_qf<FLUX, CT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+        hipLaunchKernelGGL((k_stage_qf<FLUX, CT>), dim3(grid_blocks(a)), dim3(Quad<3>::NT), lds, s, a);
+        return;
+    }
     static bool opted = false;  // above 64 KiB the kernel must opt in
     if (!opted) {
         opted = hipFuncSetAttribute((const void*)k_stage_pz<3, FLUX, CT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Pz<3>::lds(CT)) == hipSuccess;
@@ -1691,8 +1703,9 @@ static void launch_stage_pz_f(const StageArgs& a, hipStream_t s) {
 int launch_stage(int P, int flux, int prec, int block, const StageArgs& a, void* stream) {
     hipStream_t s = (hipStream_t)stream;
     if (prec == RKDG_PREC_BF16_MFMA) {
-        // BF16 contractions: staged tiles of 256 elements, one lane per element (P1, P2)
-        if (!a.staged || block != px_block(P)) return (int)hipErrorInvalidValue;
+        // BF16 contractions: staged tiles of 256 elements, one lane per element, or (P3) the
+        // four-lanes-per-element tiles
+        if (!(a.quad && P == 3) && (!a.staged || block != px_block(P))) return (int)hipErrorInvalidValue;
         switch (P) {
             case 1: launch_stage_px_p<1, CT_BF16>(flux, a, s); break;
             case 2: launch_stage_px_p<2, CT_BF16>(flux, a, s); break;
@@ -1705,9 +1718,9 @@ int launch_stage(int P, int flux, int prec, int block, const StageArgs& a, void*
         return (int)hipGetLastError();
     }
     if (prec == RKDG_PREC_FP32_MFMA) {
-        // staged tiles of 256 elements, one lane per element (P1, P2)
-        if (a.staged) {
-            if (block != px_block(P)) return (int)hipErrorInvalidValue;
+        // staged tiles of 256 elements, one lane per element, or (P3) four lanes per element
+        if (a.staged || a.quad) {
+            if (a.quad ? P != 3 : block != px_block(P)) return (int)hipErrorInvalidValue;
             switch (P) {
                 case 1: launch_stage_px_p<1, CT_F32>(flux, a, s); break;
                 case 2: launch_stage_px_p<2, CT_F32>(flux, a, s); break;

@@ -1,7 +1,7 @@
-"""The four-lanes-per-element FP64 form (P3, Roe, and LF on small meshes) at the sizes where its
-tiles can go wrong: partial tiles of 16 elements per wave and 64 or 128 per workgroup, tiles whose
-edges are all boundary or halo edges, and a caller order it must leave to
-the general kernel.  Against the oracle at the FP64 bar (1e-12)."""
+"""The four-lanes-per-element forms (FP64 at P3, with Roe, and for LF on small meshes; the
+precision forms at P3) at the sizes where their tiles can go wrong: partial tiles of 16 elements
+per wave and 64 or 128 per workgroup, tiles whose edges are all boundary or halo edges, and a
+caller order they must leave to the general kernels.  Against the oracle, FP64 at 1e-12."""
 import numpy as np
 import pytest
 
@@ -41,6 +41,34 @@ def test_tile_remainders(P, flux, bc):
         err = rel_l2(s.get_state(), o.get_state(), o.mass())
         assert np.all(err < TOL), (nx, ny, err)
         assert np.allclose(s.residual(), o.residual_change(), rtol=1e-9, atol=1e-14)
+        s.close()
+
+
+# Three steps at CFL 0.1 move a mode by at most about its deviation (0.06 over the modes, 0.2 the
+# smallest mean): bf16 rounds each by 2^-9 twice, 3 * 0.3 * 0.06 * 2^-8 / 0.2 = 1e-3; FP32 rounds
+# point values and fluxes up to 3 by 2^-24, 3 * 0.3 * 3 * 2^-24 / 0.2 = 8e-7.
+@pytest.mark.parametrize("prec,tol", [("fp32", 1e-6), ("bf16", 1e-3)])
+@pytest.mark.parametrize("flux", ["lf", "roe"])
+@pytest.mark.parametrize("bc", [0, BC_FARFIELD, BC_OUTFLOW, BC_REFLECTION])
+def test_p3_precision_tile_remainders(bc, flux, prec, tol):
+    """The P3 precision form's tiles at the same sizes, and (the last) a row-major order whose tiles
+    hold more halo edges than the form admits."""
+    for nx, ny, row_major in [(*n, False) for n in SIZES] + [(32, 12, True), (44, 12, True)]:
+        if bc == 0 and min(nx, ny) < 3:
+            continue
+        print(f"case: P3 {prec} tiles {flux} bc {bc} {nx}x{ny} row-major {row_major}", flush=True)
+        g = Grid.splitquad(nx, ny, 0.0, 0.0, 10.0, 10.0 * ny / nx, periodic=bc == 0, diagonal=1, jitter=0.2, seed=nx,
+                           bc=bc or BC_OUTFLOW)
+        kw = dict(order=np.arange(g.n_elements, dtype=np.int32)) if row_major else {}
+        o, _ = make_pair(g, P=3, flux=flux, dt_policy="max", cfl=0.1, freestream=[1.0, 0.3, 0.2, 2.6])
+        s = Solver(g, degree=3, flux=flux, dt_policy="max", cfl=0.1, freestream=[1.0, 0.3, 0.2, 2.6], precision=prec, **kw)
+        s.set_state(noisy_state(s, nx), basis=1)
+        o.set_state(s.get_state())
+        s.advance(3)
+        o.advance(3)
+        err = rel_l2(s.get_state(), o.get_state(), o.mass())
+        assert np.all(err < tol), (nx, ny, err)
+        assert np.all(err > 0)
         s.close()
 
 
