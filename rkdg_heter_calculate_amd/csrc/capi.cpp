@@ -367,8 +367,11 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     if (c->block % 64 || c->block < 64 || c->block > 256) { delete c; return fail(nullptr, RKDG_ERR_ARG, "block must be 64..256, multiple of 64"); }
     // FP64 without a caller block or a switch among the one-lane-per-element forms: four lanes
     // per element (k_stage_q) at P3, with Roe, and for LF on meshes too small for the
-    // one-lane forms (quad_max_lf).  RKDG_QUAD=0: never, 1: always.
-    const bool want_quad = prm->precision == RKDG_PREC_FP64 && prm->block == 0 && !std::getenv("RKDG_BLOCK") &&
+    // one-lane forms (quad_max_lf).  RKDG_QUAD=0: never, 1: always.  Where its tiles are the
+    // smaller ones (P1, P2: 64 elements against 256), only up to the tiles that the
+    // allocation-free step accepts: 4.2M elements, above which it would refuse the mesh.
+    const bool noalloc_fits = c->block <= quad_block(c->P) || (c->E - 1) / quad_block(c->P) < NOALLOC_MAX_TILES;
+    const bool want_quad = prm->precision == RKDG_PREC_FP64 && prm->block == 0 && noalloc_fits && !std::getenv("RKDG_BLOCK") &&
                            !std::getenv("RKDG_STAGED") && !std::getenv("RKDG_PIPE") && !std::getenv("RKDG_PERSIST") &&
                            env_int("RKDG_QUAD", c->P == 3 || prm->flux == RKDG_FLUX_ROE || c->E <= quad_max_lf(c->P));
     c->xcd_remap = env_int("RKDG_XCD_REMAP", 1);

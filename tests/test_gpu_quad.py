@@ -5,7 +5,9 @@ caller order they must leave to the general kernels.  Against the oracle, FP64 a
 import numpy as np
 import pytest
 
-from rkdg_heter_calculate_amd import BASIS_NATIVE, BC_FARFIELD, BC_OUTFLOW, BC_REFLECTION, Batch, Grid, Solver
+from rkdg_heter_calculate_amd import (BASIS_NATIVE, BC_FARFIELD, BC_OUTFLOW, BC_REFLECTION, IC_VORTEX, Batch, Grid,
+                                      Solver, vortex_params)
+from rkdg_heter_calculate_amd import _lib as L
 from helpers import make_pair, rel_l2, vortex_grid, vortex_ic
 
 pytestmark = pytest.mark.gpu
@@ -153,3 +155,15 @@ def test_batch_instances_equal_single_meshes(P, flux):
     with pytest.raises(Exception):  # chosen by the library, not through set_tiles
         b.set_tiles(2, b.tiles()["block"], 0)
     b.close()
+
+
+def test_the_allocation_free_step_takes_meshes_above_the_small_tiles_limit():
+    """4,194,304 elements fill the allocation-free step's 65,536 tiles at 64 elements per tile; a
+    larger mesh runs the 256-element tiles and is accepted."""
+    print("case: step_noalloc P1 Roe 4,199,202 triangles", flush=True)
+    s = Solver(Grid.splitquad(1449, 1449, 0.0, 0.0, 10.0, 10.0, periodic=True), degree=1, flux="roe", dt_policy="max", cfl=0.3)
+    s.project_ic(IC_VORTEX, vortex_params())
+    dt = s.compute_dt()
+    L.check(L.load().rkdg_step_noalloc(s.h, dt, None, None), s.h, "step_noalloc")
+    assert np.all(np.isfinite(s.get_state(basis=1)))
+    s.close()
