@@ -150,7 +150,9 @@ int rkdg_residual(rkdg_ctx* ctx, double res[2]);
  * is rejected with RKDG_ERR_ARG.  res_dev (device memory, may be NULL) receives the step's
  * residual pair, as rkdg_residual reports it.  The context's simulated time and step count
  * do not advance and non-physical states are not reported (nothing is read back).  Calls
- * share their GPU's scratch: calls that overlap on one GPU race. */
+ * share their GPU's scratch: calls that overlap on one GPU race.  With a stream of the caller's,
+ * wait for it before any other call on ctx: those use the context's stage buffers (rkdg_get_state
+ * forms the caller's order in one). */
 #define RKDG_NOALLOC_MAX_TILES 65536
 int rkdg_step_noalloc(rkdg_ctx* ctx, double dt, double* res_dev, void* stream);
 
