@@ -1334,8 +1334,11 @@ __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
             for (int i = 3; i < Np; ++i) c[v][i] = 0.0;
         }
     }
-    // bounds over all points: rho >= rlo, |m| <= mhi, rho E >= elo, hence p >= plo.  Beyond the
-    // margin (rounding is 1e-15 of the mean) no point is below POS_EPS and nothing is scaled.
+    // bounds over all points: rho >= rlo, |m| <= (m1, m2), rho E >= elo, hence p >= plo.  The sums
+    // are rounded to 1e-15 of the mean, which at rlo >= 1e-3 of it is 1e-12 of rlo and of the
+    // kinetic energy, and that is below rho E where plo is positive: beyond the margins, 100 times
+    // as large, no point is below POS_EPS and nothing is scaled.  (Nearer to vacuum plo's own
+    // rounding reaches the pressure: every point is looked at.)
     const double g = a.gamma;
     bool scale;
     {
@@ -1347,7 +1350,7 @@ __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
         const double rlo = c[0][0] - dev[0], elo = c[3][0] - dev[3];
         const double m1 = fabs(c[1][0]) + dev[1], m2 = fabs(c[2][0]) + dev[2];
         const double plo = (g - 1.0) * (elo - 0.5 * (m1 * m1 + m2 * m2) * frcp(rlo));
-        scale = !(rlo > fmax(1e-10 * c[0][0], 2 * POS_EPS) && plo > fmax(1e-10 * c[3][0], 2 * POS_EPS));
+        scale = !(rlo > fmax(1e-3 * c[0][0], 2 * POS_EPS) && plo > fmax(1e-10 * c[3][0], 2 * POS_EPS));
     }
     if (scale) {
         // positivity: density first, then pressure, at every volume and edge point
