@@ -232,6 +232,7 @@ struct LimArgs {
     const DevState* st;
     int slot;
     double t_end;
+    int warm;              // some workgroups take the positivity loop in any case (launch_limiter)
 };
 
 // Staged form: tiles of staged_block(P) elements whose LDS image has rows of

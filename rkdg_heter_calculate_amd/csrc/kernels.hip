@@ -1248,8 +1248,6 @@ __global__ void k_state_init(DevState* st, int n, int slot, double t) {
 // the positivity-preserving scaling of Zhang & Shu (2010), in place.  The limiter reads
 // the neighbours' means only and never modifies a mean, so the in-place update is
 // race-free.  Flags: bit 0 TVB-limited, bit 1 positivity-scaled.
-constexpr double POS_EPS = 1e-13;
-
 //
 // Bound: the bytes of the state it reads.  Most elements of a flow need neither half of it, so
 // each is entered only by elements that may: a component whose midpoint deviations are all
@@ -1257,6 +1255,16 @@ constexpr double POS_EPS = 1e-13;
 // neighbours and no limiter geometry (60 of 172 bytes at P1); and a bound on density and
 // pressure over all points at once (sums of |mode| times the largest |psi|) rules the
 // positivity loop (16 points and divisions at P1) out.
+//
+// On meshes of a few waves per SIMD the time is that of the waves that enter both halves, and much
+// of theirs is fetching instructions no other wave has run in the launch (clock stamps at 131,072
+// triangles, P1: 11,500 cycles in the first half and 6,000 in the second, 3,200 where other waves
+// had been through it).  So the first half is one copy of its code for the four components (their
+// modes and means take turns in row 0): 32,768 triangles, four-quadrant problem, P1 11.9 -> 10.8 us
+// per launch, P2 14.2 -> 13.2; where every element is limited 9.3 -> 8.2 and 10.3 -> 9.2; and a.warm
+// sends every third workgroup of an XCD through the second half (launch_limiter).
+constexpr double POS_EPS = 1e-13;
+
 template <int P>
 __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
     using D = Deg<P>;
@@ -1295,44 +1303,63 @@ __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
 #pragma unroll
         for (int r = 0; r < 6; ++r) al[r] = tmx(a.lim, r, LIM_ROWS, e);
         const int pk = a.pairs[e];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const double m0 = c[v][0];
+        int limited = 0;  // components, a bit each
+#pragma unroll 1
+        for (int v = 0; v < 4; ++v) {  // component v is in row 0
+            const double m0 = c[0][0];
             double d[3];
             bool changed = false;
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const double ut = T.Vmid[k][1] * c[v][1] + T.Vmid[k][2] * c[v][2];
+                const double ut = T.Vmid[k][1] * c[0][1] + T.Vmid[k][2] * c[0][2];
                 const int k1 = (pk >> (4 * k)) & 3, k2 = (pk >> (4 * k + 2)) & 3;
-                double n1 = nm[0][v], n2 = nm[0][v];
-                if (k1 == 1) n1 = nm[1][v]; else if (k1 == 2) n1 = nm[2][v];
-                if (k2 == 1) n2 = nm[1][v]; else if (k2 == 2) n2 = nm[2][v];
+                const double n1 = k1 == 1 ? nm[1][0] : (k1 == 2 ? nm[2][0] : nm[0][0]);
+                const double n2 = k2 == 1 ? nm[1][0] : (k2 == 2 ? nm[2][0] : nm[0][0]);
                 const double b = nu * (al[2 * k] * (n1 - m0) + al[2 * k + 1] * (n2 - m0));
-                double r;
+                double r = 0.0;
+                if (ut > 0 && b > 0) r = fmin(ut, b);
+                if (ut < 0 && b < 0) r = fmax(ut, b);
                 if (fabs(ut) <= tol) r = ut;
-                else if (ut > 0 && b > 0) r = fmin(ut, b);
-                else if (ut < 0 && b < 0) r = fmax(ut, b);
-                else r = 0.0;
-                if (r != ut) changed = true;
+                changed |= r != ut;
                 d[k] = r;
             }
-            if (!changed) continue;
-            flag = 1;
-            const double sum = d[0] + d[1] + d[2];
-            if (sum != 0.0) {
-                double pos = 0, neg = 0;
+            if (changed) {
+                limited |= 1 << v;
+                const double sum = d[0] + d[1] + d[2];
+                if (sum != 0.0) {
+                    double pos = 0, neg = 0;
 #pragma unroll
-                for (int k = 0; k < 3; ++k) { pos += fmax(0.0, d[k]); neg += fmax(0.0, -d[k]); }
-                const double tp = pos > 0 ? fmin(1.0, neg / pos) : 0.0;
-                const double tn = neg > 0 ? fmin(1.0, pos / neg) : 0.0;
+                    for (int k = 0; k < 3; ++k) { pos += fmax(0.0, d[k]); neg += fmax(0.0, -d[k]); }
+                    const double tp = pos > 0 ? fmin(1.0, neg / pos) : 0.0;
+                    const double tn = neg > 0 ? fmin(1.0, pos / neg) : 0.0;
 #pragma unroll
-                for (int k = 0; k < 3; ++k) d[k] = tp * fmax(0.0, d[k]) - tn * fmax(0.0, -d[k]);
+                    for (int k = 0; k < 3; ++k) d[k] = tp * fmax(0.0, d[k]) - tn * fmax(0.0, -d[k]);
+                }
+                c[0][1] = T.recon[0][0] * d[0] + T.recon[0][1] * d[1] + T.recon[0][2] * d[2];
+                c[0][2] = T.recon[1][0] * d[0] + T.recon[1][1] * d[1] + T.recon[1][2] * d[2];
             }
-            c[v][1] = T.recon[0][0] * d[0] + T.recon[0][1] * d[1] + T.recon[0][2] * d[2];
-            c[v][2] = T.recon[1][0] * d[0] + T.recon[1][1] * d[1] + T.recon[1][2] * d[2];
+            // the next component into row 0 (after four turns every row is back)
 #pragma unroll
-            for (int i = 3; i < Np; ++i) c[v][i] = 0.0;
+            for (int i = 0; i < 3; ++i) {
+                const double t = c[0][i];
+                c[0][i] = c[1][i];
+                c[1][i] = c[2][i];
+                c[2][i] = c[3][i];
+                c[3][i] = t;
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                nm[k][0] = nm[k][1];
+                nm[k][1] = nm[k][2];
+                nm[k][2] = nm[k][3];
+            }
         }
+        if (limited) flag = 1;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int i = 3; i < Np; ++i)
+                if (limited >> v & 1) c[v][i] = 0.0;
     }
     // bounds over all points: rho >= rlo, |m| <= (m1, m2), rho E >= elo, hence p >= plo.  The sums
     // are rounded to 1e-15 of the mean, which at rlo >= 1e-3 of it is 1e-12 of rlo and of the
@@ -1351,6 +1378,7 @@ __global__ void __launch_bounds__(256) k_limit(LimArgs a) {
         const double m1 = fabs(c[1][0]) + dev[1], m2 = fabs(c[2][0]) + dev[2];
         const double plo = (g - 1.0) * (elo - 0.5 * (m1 * m1 + m2 * m2) * frcp(rlo));
         scale = !(rlo > fmax(1e-3 * c[0][0], 2 * POS_EPS) && plo > fmax(1e-10 * c[3][0], 2 * POS_EPS));
+        scale |= a.warm && (blockIdx.x >> 3) % 3 == 0;
     }
     if (scale) {
         // positivity: density first, then pressure, at every volume and edge point
@@ -1841,8 +1869,16 @@ int launch_state_init(DevState* st, int slot, double t, int n, void* stream) {
     return (int)hipGetLastError();
 }
 
-int launch_limiter(int P, const LimArgs& a, int block, void* stream) {
+// a.warm at P1 and P2 on meshes of 1.5 to 2.1 waves per SIMD (1,024 of them): there the few waves
+// that enter both halves made the launch longer than one in which every wave does.  131,072
+// triangles, P2, a third of the workgroups sent / none / every wave: four-quadrant problem 15.9 /
+// 19.6 / 16.6 us, every element limited 18.5 / 15.8 / 20.1; P1 12.6 / 14.1 / 13.5 and 14.5 / 12.2 /
+// 15.3.  Below (92,450: 14.2 / 15.7 / 15.6 and 17.0 / 13.1 / 18.3) and above (147,968: 16.0 / 17.4 /
+// 19.0 and 19.6 / 16.8 / 22.2) it is no slower without.
+int launch_limiter(int P, const LimArgs& args, int block, void* stream) {
     hipStream_t s = (hipStream_t)stream;
+    LimArgs a = args;
+    a.warm = P <= 2 && a.E > 98304 && a.E <= 140000;
     dim3 grid((a.E + block - 1) / block), blk(block);
     switch (P) {
         case 1: hipLaunchKernelGGL(k_limit<1>, grid, blk, 0, s, a); break;

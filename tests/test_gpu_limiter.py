@@ -5,8 +5,8 @@ from fractions import Fraction
 import numpy as np
 import pytest
 
-from rkdg_heter_calculate_amd import BASIS_NATIVE, Solver
-from helpers import vortex_grid
+from rkdg_heter_calculate_amd import BASIS_NATIVE, Grid, Solver, riemann4_params
+from helpers import make_pair, rel_l2, vortex_grid
 
 pytestmark = pytest.mark.gpu
 
@@ -50,4 +50,23 @@ def test_positivity_is_not_skipped_near_vacuum():
     f = s.flags()
     print("scaled", int((f == 2).sum()), "of", f.size, flush=True)
     assert np.all(f == 2)
+    s.close()
+
+
+@pytest.mark.parametrize("P", [1, 2])
+@pytest.mark.parametrize("nx,ny", [(256, 192), (223, 221), (250, 280), (280, 251)])
+def test_limiter_on_both_sides_of_the_warm_rule(P, nx, ny):
+    """98,304 elements and 98,566, 140,000 and 140,560: the launches in which some workgroups look at
+    every point and those in which only the elements do that may need it decide alike."""
+    print(f"case: limiter P{P} {nx}x{ny}", flush=True)
+    g = Grid.splitquad(nx, ny, 0.0, 0.0, 1.0, ny / nx, periodic=False, diagonal=1, jitter=0.2, seed=9)
+    o, s = make_pair(g, P=P, flux="lf", limiter=True, dt_policy="max", cfl=0.2 if P == 1 else 0.1, tvb_M=50.0)
+    o.project(2, riemann4_params())
+    s.set_state(o.get_state())
+    s.advance(3)
+    o.advance(3)
+    err = rel_l2(s.get_state(), o.get_state(), o.mass())
+    assert np.all(err < 1e-12), err
+    assert np.array_equal(s.flags(), o.flags())
+    assert (o.flags() != 0).sum() > 100
     s.close()
