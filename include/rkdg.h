@@ -151,8 +151,8 @@ int rkdg_residual(rkdg_ctx* ctx, double res[2]);
  * residual pair, as rkdg_residual reports it.  The context's simulated time and step count
  * do not advance and non-physical states are not reported (nothing is read back).  Calls
  * share their GPU's scratch: calls that overlap on one GPU race.  With a stream of the caller's,
- * wait for it before any other call on ctx: those use the context's stage buffers (rkdg_get_state
- * forms the caller's order in one). */
+ * wait for it before calls that change the context's state, and before reading it: rkdg_get_state
+ * and rkdg_get_flags change nothing, but what they return meanwhile is of no one stage. */
 #define RKDG_NOALLOC_MAX_TILES 65536
 int rkdg_step_noalloc(rkdg_ctx* ctx, double dt, double* res_dev, void* stream);
 

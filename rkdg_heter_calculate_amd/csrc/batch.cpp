@@ -48,6 +48,7 @@ struct rkdg_batch {
     double* cfl = nullptr;
     int* tile_mesh = nullptr;
     int* order_dev = nullptr;   // caller element of each position (state exchange)
+    double* rows = nullptr;     // caller rows of an instance's state exchange, for the largest one
     Transfer xfer;              // pinned chunks of the state transfers
     int ntiles = 0;
     long long steps = 0;
@@ -155,19 +156,20 @@ static int bwavespeed_all(rkdg_batch* b) {
     return RKDG_OK;
 }
 
-// One instance's state exchange through the first rows of U[1] (which holds no state between
-// steps: stage 0 writes all of it).
-static ExchangeArgs bexchange(rkdg_batch* b, int i, int32_t basis) {
+// One instance's state exchange, one part (exchange_vars variables).
+static int bexchange(rkdg_batch* b, int i, int32_t basis, bool out, int part) {
     ExchangeArgs x{};
     x.U = b->U[0];
-    x.rows = b->U[1];
+    x.rows = b->rows;
     x.geo = b->geo;
     x.order = b->order_dev;
     x.first = b->off[i];
     x.n = b->E[i];
-    x.pad = b->E[i];
+    x.pad = b->E[i];  // (the padding columns keep their rest state)
     x.basis = basis;
-    return x;
+    x.nv = exchange_vars(b->Np, b->E[i], basis);
+    x.v0 = part * x.nv;
+    return launch_exchange(b->P, x, out, b->stream);
 }
 
 extern "C" {
@@ -371,7 +373,10 @@ int rkdg_batch_create(int32_t n, const rkdg_mesh* meshes, const rkdg_params* par
     BCREATECHK(hipMemcpy(b->nbr, to_tile_major(hnbr, NBR_ROWS, ld).data(), sizeof(int) * hnbr.size(), hipMemcpyHostToDevice));
     BCREATECHK(hipMemcpy(b->dtflag, hflag.data(), hflag.size(), hipMemcpyHostToDevice));
     BCREATECHK(hipMemcpy(b->cfl, hcfl.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-    b->bytes = sizeof(int) * (size_t)ld + 3 * ub + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size();
+    size_t rows = 0;
+    for (int i = 0; i < n; ++i) rows = std::max(rows, exchange_bytes(b->Np, b->E[i]));
+    BCREATECHK(hipMalloc(&b->rows, rows));
+    b->bytes = sizeof(int) * (size_t)ld + rows + 3 * ub + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size();
     const bool prec_form = p0.precision != RKDG_PREC_FP64;
     if (!prec_form && env_int("RKDG_QUAD", 1)) {
         std::vector<int> list;
@@ -459,7 +464,7 @@ int rkdg_batch_destroy(rkdg_batch* b) {
     if (b->graph2) hipGraphExecDestroy(b->graph2);
     for (int k = 0; k < 3; ++k) hipFree(b->U[k]);
     hipFree(b->geo); hipFree(b->nbr); hipFree(b->dtflag); hipFree(b->st); hipFree(b->cfl); hipFree(b->tile_mesh);
-    hipFree(b->order_dev);
+    hipFree(b->order_dev); hipFree(b->rows);
     transfer_free(b->xfer);
     hipFree(b->qlist);
     hipFree(b->nloc); hipFree(b->hoff); hipFree(b->hids);
@@ -471,12 +476,9 @@ int rkdg_batch_destroy(rkdg_batch* b) {
 int rkdg_batch_set_state(rkdg_batch* b, int32_t i, int32_t basis, const double* U) {
     if (!b || i < 0 || i >= b->n || !U) return bfail(b, RKDG_ERR_ARG, "batch_set_state");
     BCHK(b, hipSetDevice(b->dev));
-    const int E = b->E[i], Np = b->Np, P = b->P;
-    // the instance's layout tiles are one contiguous block of the tile-major state; its
-    // padding columns keep their rest state, so the block is read, updated and written back
-    // (U[1] holds no state between steps; the instance's padding columns keep their rest state)
-    BCHK(b, (hipError_t)copy_to_device(b->xfer, b->stream, b->U[1], U, sizeof(double) * 4 * Np * (size_t)E));
-    const int xrc = launch_exchange(b->P, bexchange(b, i, basis), false, b->stream);
+    const int xrc = copy_to_device(b->xfer, b->stream, b->rows, U, exchange_part(b->Np, b->E[i], basis),
+                                   4 / exchange_vars(b->Np, b->E[i], basis),
+                                   [&](int part) { return bexchange(b, i, basis, false, part); });
     if (xrc) return bfail(b, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(xrc));
     int rc = bwavespeed_all(b);
     if (rc) return rc;
@@ -487,10 +489,10 @@ int rkdg_batch_set_state(rkdg_batch* b, int32_t i, int32_t basis, const double* 
 int rkdg_batch_get_state(rkdg_batch* b, int32_t i, int32_t basis, double* U) {
     if (!b || i < 0 || i >= b->n || !U) return bfail(b, RKDG_ERR_ARG, "batch_get_state");
     BCHK(b, hipSetDevice(b->dev));
-    const int E = b->E[i], Np = b->Np;
-    const int xrc = launch_exchange(b->P, bexchange(b, i, basis), true, b->stream);
+    const int xrc = copy_to_host(b->xfer, b->stream, U, b->rows, exchange_part(b->Np, b->E[i], basis),
+                                 4 / exchange_vars(b->Np, b->E[i], basis),
+                                 [&](int part) { return bexchange(b, i, basis, true, part); });
     if (xrc) return bfail(b, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(xrc));
-    BCHK(b, (hipError_t)copy_to_host(b->xfer, b->stream, U, b->U[1], sizeof(double) * 4 * Np * (size_t)E));
     return RKDG_OK;
 }
 

@@ -158,6 +158,7 @@ struct rkdg_ctx {
     long long ld = 0;
     std::vector<int32_t> order, pos;  // order[p] = caller id at device position p
     int* order_dev = nullptr;         // the same on the device (state exchange)
+    double* rows = nullptr;           // caller rows of the state exchange (exchange_bytes)
     Transfer xfer;                    // pinned chunks of the state transfers
     std::vector<double> ex, ey;       // [E][3] element vertex coordinates (caller order)
     double* U[3] = {nullptr, nullptr, nullptr};
@@ -570,9 +571,10 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     CREATECHK(hipMalloc(&c->dtflag, hflag.size()));
     CREATECHK(hipMalloc(&c->flags, sizeof(int) * ld));
     CREATECHK(hipMalloc(&c->order_dev, sizeof(int) * E));
+    CREATECHK(hipMalloc(&c->rows, exchange_bytes(c->Np, E)));
     CREATECHK(hipMalloc(&c->st, sizeof(DevState)));
     CREATECHK(hipMalloc(&c->res_part, sizeof(double) * 2 * c->ntiles));
-    c->bytes = sizeof(int) * (size_t)E + 3 * ubytes + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size() + sizeof(int) * ld +
+    c->bytes = sizeof(int) * (size_t)E + exchange_bytes(c->Np, E) + 3 * ubytes + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size() + sizeof(int) * ld +
                sizeof(double) * 2 * c->ntiles;
     for (int b = 0; b < 3; ++b) CREATECHK(hipMemsetAsync(c->U[b], 0, ubytes, c->stream));
     CREATECHK(hipMemsetAsync(c->flags, 0, sizeof(int) * ld, c->stream));
@@ -625,7 +627,7 @@ int rkdg_destroy(rkdg_ctx* c) {
     for (int b = 0; b < 3; ++b) hipFree(c->U[b]);
     hipFree(c->geo); hipFree(c->nbr); hipFree(c->dtflag); hipFree(c->lim); hipFree(c->pairs);
     hipFree(c->nloc); hipFree(c->hoff); hipFree(c->hids);
-    hipFree(c->order_dev);
+    hipFree(c->order_dev); hipFree(c->rows);
     transfer_free(c->xfer);
     hipFree(c->flags); hipFree(c->st); hipFree(c->res_part);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -633,26 +635,28 @@ int rkdg_destroy(rkdg_ctx* c) {
     return RKDG_OK;
 }
 
-// State exchange: the caller's rows pass through a stage buffer that holds no state (one of
-// U[1], U[2]: only the step-start buffer and, inside a step, the latest stage are live).
-static ExchangeArgs exchange_args(rkdg_ctx* c, double* U, double* rows, int32_t basis) {
+// State exchange of U, one part (exchange_vars variables).
+static int exchange(rkdg_ctx* c, double* U, int32_t basis, bool out, int part) {
     ExchangeArgs x{};
     x.U = U;
-    x.rows = rows;
+    x.rows = c->rows;
     x.geo = c->geo;
     x.order = c->order_dev;
     x.first = 0;
     x.n = c->E;
     x.pad = (int)c->ld;
     x.basis = basis;
-    return x;
+    x.nv = exchange_vars(c->Np, c->E, basis);
+    x.v0 = part * x.nv;
+    return launch_exchange(c->P, x, out, c->stream);
 }
 
 int rkdg_set_state(rkdg_ctx* c, int32_t basis, const double* U) {
     if (!c || !U || (basis != RKDG_BASIS_ELEMENT && basis != RKDG_BASIS_NATIVE)) return fail(c, RKDG_ERR_ARG, "set_state");
     HIPCHK(c, hipSetDevice(c->dev));
-    HIPCHK(c, (hipError_t)copy_to_device(c->xfer, c->stream, c->U[1], U, sizeof(double) * 4 * c->Np * (size_t)c->E));
-    int rc = launch_exchange(c->P, exchange_args(c, c->U[0], c->U[1], basis), false, c->stream);
+    int rc = copy_to_device(c->xfer, c->stream, c->rows, U, exchange_part(c->Np, c->E, basis),
+                            4 / exchange_vars(c->Np, c->E, basis),
+                            [&](int part) { return exchange(c, c->U[0], basis, false, part); });
     if (rc) return fail(c, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(rc));
     c->cur = 0;
     c->next_stage = 0;
@@ -667,10 +671,10 @@ int rkdg_set_state(rkdg_ctx* c, int32_t basis, const double* U) {
 int rkdg_get_state(rkdg_ctx* c, int32_t basis, double* U) {
     if (!c || !U || (basis != RKDG_BASIS_ELEMENT && basis != RKDG_BASIS_NATIVE)) return fail(c, RKDG_ERR_ARG, "get_state");
     HIPCHK(c, hipSetDevice(c->dev));
-    double* rows = c->U[c->cur == 1 ? 2 : 1];
-    const int rc = launch_exchange(c->P, exchange_args(c, c->U[c->cur], rows, basis), true, c->stream);
+    const int rc = copy_to_host(c->xfer, c->stream, U, c->rows, exchange_part(c->Np, c->E, basis),
+                                4 / exchange_vars(c->Np, c->E, basis),
+                                [&](int part) { return exchange(c, c->U[c->cur], basis, true, part); });
     if (rc) return fail(c, RKDG_ERR_HIP, std::string("state exchange: ") + hip_error_string(rc));
-    HIPCHK(c, (hipError_t)copy_to_host(c->xfer, c->stream, U, rows, sizeof(double) * 4 * c->Np * (size_t)c->E));
     return RKDG_OK;
 }
 
@@ -911,10 +915,9 @@ int rkdg_time(rkdg_ctx* c, double* t, int64_t* steps) {
 int rkdg_get_flags(rkdg_ctx* c, int32_t* flags) {
     if (!c || !flags) return fail(c, RKDG_ERR_ARG, "get_flags");
     HIPCHK(c, hipSetDevice(c->dev));
-    int* rows = (int*)c->U[c->cur == 1 ? 2 : 1];  // holds no state (exchange_args)
-    const int rc = launch_flags_out(c->flags, c->order_dev, c->E, rows, c->stream);
+    const int rc = copy_to_host(c->xfer, c->stream, flags, c->rows, sizeof(int) * (size_t)c->E, 1,
+                                [&](int) { return launch_flags_out(c->flags, c->order_dev, c->E, (int*)c->rows, c->stream); });
     if (rc) return fail(c, RKDG_ERR_HIP, std::string("flags: ") + hip_error_string(rc));
-    HIPCHK(c, (hipError_t)copy_to_host(c->xfer, c->stream, flags, rows, sizeof(int) * (size_t)c->E));
     return RKDG_OK;
 }
 

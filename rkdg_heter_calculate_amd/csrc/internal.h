@@ -96,9 +96,13 @@ struct Transfer {
     char* pin = nullptr;
     size_t bytes = 0;
 };
-// Synchronous copies ordered behind the stream's work; return a hipError_t.
-int copy_to_host(Transfer& t, void* stream, void* host, const void* dev, size_t n);
-int copy_to_device(Transfer& t, void* stream, void* dev, const void* host, size_t n);
+// Synchronous copies ordered behind the stream's work, of parts of n bytes each: consecutive on
+// the host, all through the device buffer dev.  form(p) launches what writes part p into dev, use(p)
+// what takes it out; they and the copies return a hipError_t.
+int copy_to_host(Transfer& t, void* stream, void* host, const void* dev, size_t n, int parts,
+                 const std::function<int(int)>& form);
+int copy_to_device(Transfer& t, void* stream, void* dev, const void* host, size_t n, int parts,
+                   const std::function<int(int)>& use);
 void transfer_free(Transfer& t);
 
 // Host-side basis/geometry helpers (basis.cpp)
@@ -275,9 +279,9 @@ constexpr long long quad_lds_bytes(int P) {
 
 int upload_tables(int P, const DevTables& t);  // per current device
 // State exchange on the device: the tile-major state of n elements from device position first
-// (U: the whole array) <-> caller rows [4 Np][n] in the caller's element order and basis.
-// order[first + i]: the caller element at that position.  On the way in the positions up to pad
-// (at least n) of them are cleared.
+// (U: the whole array) <-> caller rows [nv Np][n] in the caller's element order and basis, of the
+// nv (1 or 4) variables from v0.  order[first + i]: the caller element at that position.  On the
+// way in the positions up to pad (at least n) of them are cleared.
 struct ExchangeArgs {
     double* U;
     double* rows;
@@ -285,8 +289,19 @@ struct ExchangeArgs {
     const int* order;
     int first, n, pad;
     int basis;             // RKDG_BASIS_*
+    int v0, nv;
 };
 int launch_exchange(int P, const ExchangeArgs& a, bool out, void* stream);  // out: U -> rows
+// The rows have a buffer of their own (a read leaves every state buffer alone, also one that a
+// caller's stream still works on).  A state of more than the pinned chunks hold crosses one variable
+// at a time, in a quarter of the space and no slower; in the element basis of P3 all at once,
+// because each part builds that basis anew (2.1M triangles: 2.6 ms, to the device 24.4 ms in four
+// parts against 16.5).
+constexpr int exchange_vars(int Np, long long n, int basis) {
+    return 32LL * Np * n <= 32LL << 20 || (Np == 10 && basis == RKDG_BASIS_ELEMENT) ? 4 : 1;
+}
+constexpr size_t exchange_part(int Np, long long n, int basis) { return (size_t)8 * Np * n * exchange_vars(Np, n, basis); }
+constexpr size_t exchange_bytes(int Np, long long n) { return exchange_part(Np, n, RKDG_BASIS_ELEMENT); }
 int launch_flags_out(const int* flags, const int* order, int n, int* out, void* stream);
 int launch_stage(int P, int flux, int prec, int block, const StageArgs& a, void* stream);
 int launch_wavespeed(int P, const StageArgs& a, int block, void* stream);

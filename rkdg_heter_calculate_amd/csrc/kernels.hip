@@ -1487,21 +1487,24 @@ struct ExchangeBasis {
     }
 };
 
-// Tile-major state -> the caller's rows [4 Np][n], one lane per element (a 2.1M-triangle P3 state
-// in the native basis: about 1.5 ms of the 17-30 ms its 671 MB take to the host).
-template <int P, int BASIS>
+// Tile-major state -> the caller's rows, one lane per element (a 2.1M-triangle P3 state in the
+// native basis: about 1.5 ms of the 17-30 ms its 671 MB take to the host).
+template <int P, int BASIS, int NV>
 __global__ void __launch_bounds__(256) k_state_out(ExchangeArgs a) {
     constexpr int Np = Deg<P>::Np;
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= a.n) return;
     const int e = a.first + i, to = a.order[e];
-    double u[4][Np];
-    load_modes<Np>(a.U, e, u);
+    double u[NV][Np];
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int k = 0; k < Np; ++k) u[v][k] = tmx(a.U, (a.v0 + v) * Np + k, 4 * Np, e);
     if constexpr (BASIS == RKDG_BASIS_ELEMENT) {
         ExchangeBasis<P> B;
         B.build(a.geo, e);
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+        for (int v = 0; v < NV; ++v)
 #pragma unroll
             for (int k = 0; k < Np; ++k) {
                 double s = 0.0;
@@ -1511,35 +1514,35 @@ __global__ void __launch_bounds__(256) k_state_out(ExchangeArgs a) {
             }
     } else {
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+        for (int v = 0; v < NV; ++v)
 #pragma unroll
             for (int k = 0; k < Np; ++k) a.rows[(size_t)(v * Np + k) * a.n + to] = u[v][k];
     }
 }
 
 // The caller's rows -> tile-major state; positions past the elements are cleared.
-template <int P, int BASIS>
+template <int P, int BASIS, int NV>
 __global__ void __launch_bounds__(256) k_state_in(ExchangeArgs a) {
     constexpr int Np = Deg<P>::Np;
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= a.pad) return;
     const int e = a.first + i;
-    double u[4][Np];
+    double u[NV][Np];
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
+    for (int v = 0; v < NV; ++v)
 #pragma unroll
         for (int k = 0; k < Np; ++k) u[v][k] = 0.0;
     if (i < a.n) {
         const int from = a.order[e];
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+        for (int v = 0; v < NV; ++v)
 #pragma unroll
             for (int k = 0; k < Np; ++k) u[v][k] = a.rows[(size_t)(v * Np + k) * a.n + from];
         if constexpr (BASIS == RKDG_BASIS_ELEMENT) {
             ExchangeBasis<P> B;
             B.build(a.geo, e);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
+            for (int v = 0; v < NV; ++v) {
                 double d[Np];
 #pragma unroll
                 for (int j = 0; j < Np; ++j) d[j] = 0.0;
@@ -1553,20 +1556,26 @@ __global__ void __launch_bounds__(256) k_state_in(ExchangeArgs a) {
         }
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
+    for (int v = 0; v < NV; ++v)
 #pragma unroll
-        for (int k = 0; k < Np; ++k) tmx(a.U, v * Np + k, 4 * Np, e) = u[v][k];
+        for (int k = 0; k < Np; ++k) tmx(a.U, (a.v0 + v) * Np + k, 4 * Np, e) = u[v][k];
+}
+
+template <int P, int BASIS, int NV>
+static void launch_exchange_pbn(const ExchangeArgs& a, bool out, hipStream_t s) {
+    const dim3 grid(((out ? a.n : a.pad) + 255) / 256), blk(256);
+    if (out) hipLaunchKernelGGL((k_state_out<P, BASIS, NV>), grid, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_state_in<P, BASIS, NV>), grid, blk, 0, s, a);
 }
 
 template <int P>
 static void launch_exchange_p(const ExchangeArgs& a, bool out, hipStream_t s) {
-    const dim3 grid(((out ? a.n : a.pad) + 255) / 256), blk(256);
     if (a.basis == RKDG_BASIS_ELEMENT) {
-        if (out) hipLaunchKernelGGL((k_state_out<P, RKDG_BASIS_ELEMENT>), grid, blk, 0, s, a);
-        else hipLaunchKernelGGL((k_state_in<P, RKDG_BASIS_ELEMENT>), grid, blk, 0, s, a);
+        if (a.nv == 4) launch_exchange_pbn<P, RKDG_BASIS_ELEMENT, 4>(a, out, s);
+        else launch_exchange_pbn<P, RKDG_BASIS_ELEMENT, 1>(a, out, s);
     } else {
-        if (out) hipLaunchKernelGGL((k_state_out<P, RKDG_BASIS_NATIVE>), grid, blk, 0, s, a);
-        else hipLaunchKernelGGL((k_state_in<P, RKDG_BASIS_NATIVE>), grid, blk, 0, s, a);
+        if (a.nv == 4) launch_exchange_pbn<P, RKDG_BASIS_NATIVE, 4>(a, out, s);
+        else launch_exchange_pbn<P, RKDG_BASIS_NATIVE, 1>(a, out, s);
     }
 }
 

@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -71,9 +72,26 @@ struct Ring {
     }
 };
 
-int copy_ring(Transfer& t, hipStream_t s, char* host, char* dev, size_t n, bool to_host) {
+// A transfer: parts of n bytes each, one after the other on the host, all through the same device
+// buffer; form puts a part into it (on the way to the host) or takes it out.
+struct Parts {
+    char* host;
+    char* dev;
+    size_t n;
+    int parts;
+    const std::function<int(int)>& form;
+    bool to_host;
+};
+
+int copy_ring(Transfer& t, hipStream_t s, const Parts& x) {
     const int B = Transfer::CHUNKS;
-    const long long nch = (long long)((n + CHUNK - 1) / CHUNK);
+    const bool to_host = x.to_host;
+    const long long per = (long long)((x.n + CHUNK - 1) / CHUNK), nch = x.parts * per;  // chunks of a part, of all
+    auto chunk = [&](long long c, size_t& hoff, size_t& doff) {
+        doff = (size_t)(c % per) * CHUNK;
+        hoff = (size_t)(c / per) * x.n + doff;
+        return std::min(CHUNK, x.n - doff);
+    };
     const int workers = std::max(1, std::min(8, host_threads()));
     Ring r(nch, workers);
     std::vector<hipEvent_t> ev(B, nullptr);
@@ -84,11 +102,12 @@ int copy_ring(Transfer& t, hipStream_t s, char* host, char* dev, size_t n, bool 
     auto work = [&](int w) {
         for (long long c = 0; c < nch; ++c) {
             if (!r.wait_open(c)) return;
-            const size_t o = (size_t)c * CHUNK, len = std::min(CHUNK, n - o);
+            size_t o, d;
+            const size_t len = chunk(c, o, d);
             const size_t a = len * w / workers / 64 * 64, b = w == workers - 1 ? len : len * (w + 1) / workers / 64 * 64;
             char* p = t.pin + (size_t)(c % B) * CHUNK;
-            if (to_host) std::memcpy(host + o + a, p + a, b - a);
-            else std::memcpy(p + a, host + o + a, b - a);
+            if (to_host) std::memcpy(x.host + o + a, p + a, b - a);
+            else std::memcpy(p + a, x.host + o + a, b - a);
             r.done(c);
         }
     };
@@ -102,11 +121,17 @@ int copy_ring(Transfer& t, hipStream_t s, char* host, char* dev, size_t n, bool 
         return -1;
     }
     auto move = [&](long long c) {
-        const size_t o = (size_t)c * CHUNK, len = std::min(CHUNK, n - o);
+        size_t o, d;
+        const size_t len = chunk(c, o, d);
         char* p = t.pin + (size_t)(c % B) * CHUNK;
-        rc = to_host ? hipMemcpyAsync(p, dev + o, len, hipMemcpyDeviceToHost, s)
-                     : hipMemcpyAsync(dev + o, p, len, hipMemcpyHostToDevice, s);
+        // (in stream order: a part is formed after the copies of the one before it, and taken
+        // out before the copies of the next)
+        if (to_host && c % per == 0) rc = (hipError_t)x.form((int)(c / per));
+        if (rc == hipSuccess)
+            rc = to_host ? hipMemcpyAsync(p, x.dev + d, len, hipMemcpyDeviceToHost, s)
+                         : hipMemcpyAsync(x.dev + d, p, len, hipMemcpyHostToDevice, s);
         if (rc == hipSuccess) rc = hipEventRecord(ev[c % B], s);
+        if (rc == hipSuccess && !to_host && c % per == per - 1) rc = (hipError_t)x.form((int)(c / per));
     };
     if (to_host) {
         long long issued = 0;
@@ -139,37 +164,45 @@ int copy_ring(Transfer& t, hipStream_t s, char* host, char* dev, size_t n, bool 
     return (int)rc;
 }
 
-int copy(Transfer& t, void* stream, char* host, char* dev, size_t n, bool to_host) {
+int copy(Transfer& t, void* stream, const Parts& x) {
     hipStream_t s = (hipStream_t)stream;
-    hipError_t rc;
-    if (n > 0 && reserve(t, n)) {
-        if (n > ONE_SHOT) {
-            const int e = copy_ring(t, s, host, dev, n, to_host);
+    const size_t total = x.n * x.parts;
+    char* pin = nullptr;
+    if (total > 0 && reserve(t, total)) {
+        if (total > ONE_SHOT) {
+            const int e = copy_ring(t, s, x);
             if (e >= 0) return e;
         } else {
-            if (!to_host) std::memcpy(t.pin, host, n);
-            rc = to_host ? hipMemcpyAsync(t.pin, dev, n, hipMemcpyDeviceToHost, s)
-                         : hipMemcpyAsync(dev, t.pin, n, hipMemcpyHostToDevice, s);
-            const hipError_t done = hipStreamSynchronize(s);
-            if (rc == hipSuccess) rc = done;
-            if (rc == hipSuccess && to_host) std::memcpy(host, t.pin, n);
-            return (int)rc;
+            pin = t.pin;
         }
     }
-    rc = to_host ? hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, s)
-                 : hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, s);
+    // part by part, through pinned memory if there is some
+    char* const host = pin ? pin : x.host;
+    hipError_t rc = hipSuccess;
+    if (pin && !x.to_host) std::memcpy(pin, x.host, total);
+    for (int p = 0; p < x.parts && rc == hipSuccess; ++p) {
+        if (x.to_host) rc = (hipError_t)x.form(p);
+        if (rc == hipSuccess)
+            rc = x.to_host ? hipMemcpyAsync(host + p * x.n, x.dev, x.n, hipMemcpyDeviceToHost, s)
+                           : hipMemcpyAsync(x.dev, host + p * x.n, x.n, hipMemcpyHostToDevice, s);
+        if (rc == hipSuccess && !x.to_host) rc = (hipError_t)x.form(p);
+    }
     const hipError_t done = hipStreamSynchronize(s);
-    return (int)(rc == hipSuccess ? done : rc);
+    if (rc == hipSuccess) rc = done;
+    if (rc == hipSuccess && pin && x.to_host) std::memcpy(x.host, pin, total);
+    return (int)rc;
 }
 
 }  // namespace
 
-int copy_to_host(Transfer& t, void* stream, void* host, const void* dev, size_t n) {
-    return copy(t, stream, (char*)host, (char*)const_cast<void*>(dev), n, true);
+int copy_to_host(Transfer& t, void* stream, void* host, const void* dev, size_t n, int parts,
+                 const std::function<int(int)>& form) {
+    return copy(t, stream, Parts{(char*)host, (char*)const_cast<void*>(dev), n, parts, form, true});
 }
 
-int copy_to_device(Transfer& t, void* stream, void* dev, const void* host, size_t n) {
-    return copy(t, stream, (char*)const_cast<void*>(host), (char*)dev, n, false);
+int copy_to_device(Transfer& t, void* stream, void* dev, const void* host, size_t n, int parts,
+                   const std::function<int(int)>& use) {
+    return copy(t, stream, Parts{(char*)const_cast<void*>(host), (char*)dev, n, parts, use, false});
 }
 
 void transfer_free(Transfer& t) {

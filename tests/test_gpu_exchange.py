@@ -1,11 +1,12 @@
 """State exchange on the device: caller order and both bases, transfers below and above the
 one-copy limit (1.5 MiB) and the 8 MiB chunks, reads inside a step."""
+import ctypes
 import math
 
 import numpy as np
 import pytest
 
-from rkdg_heter_calculate_amd import BASIS_ELEMENT, BASIS_NATIVE, Batch, Grid, Solver
+from rkdg_heter_calculate_amd import BASIS_ELEMENT, BASIS_NATIVE, IC_VORTEX, Batch, Grid, Solver, vortex_params
 from rkdg_heter_calculate_amd import _lib as L
 from helpers import vortex_grid
 
@@ -151,5 +152,36 @@ def test_reading_inside_a_step_changes_nothing(P, prec):
             b.flags()
     assert np.array_equal(a.get_state(BASIS_NATIVE), b.get_state(BASIS_NATIVE))
     assert np.array_equal(a.flags(), b.flags())
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("P,limiter,n", [(2, False, 64), (1, True, 48), (3, False, 170)])
+def test_reading_beside_steps_on_another_stream_changes_nothing(P, limiter, n):
+    """get_state and flags while rkdg_step_noalloc works on a caller's stream: what they return is of
+    no one stage, but the steps must come out as if unread (the rows have a buffer of their own; at
+    P3 here the state crosses one variable at a time)."""
+    print(f"case: exchange beside steps P{P}", flush=True)
+    lib, hip = L.load(), ctypes.CDLL("libamdhip64.so")
+    g = vortex_grid(n, jitter=0.2, diagonal=1, seed=3)
+    kw = dict(degree=P, flux="roe", dt_policy="max", cfl=0.1, limiter=limiter)
+    a, b = Solver(g, **kw), Solver(g, **kw)
+    for s in (a, b):
+        s.project_ic(IC_VORTEX, vortex_params())
+    dt = a.compute_dt()
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0
+    for _ in range(4):
+        for _ in range(100):
+            L.check(lib.rkdg_step_noalloc(b.h, dt, None, stream), b.h, "step_noalloc")
+        for _ in range(5):
+            b.get_state(BASIS_ELEMENT)
+            b.flags()
+        assert hip.hipStreamSynchronize(stream) == 0
+        for _ in range(100):
+            L.check(lib.rkdg_step_noalloc(a.h, dt, None, None), a.h, "step_noalloc")
+        assert np.array_equal(a.get_state(BASIS_NATIVE), b.get_state(BASIS_NATIVE))
+        assert np.array_equal(a.flags(), b.flags())
+    assert hip.hipStreamDestroy(stream) == 0
     a.close()
     b.close()
