@@ -90,7 +90,8 @@ void parallel_for(int n, const std::function<void(int, int)>& body);
 int host_threads();  // its threads at most (RKDG_HOST_THREADS)
 
 // Pinned chunks for state transfers (transfer.cpp), kept with the context or batch that owns
-// them: at most CHUNKS of 8 MiB, allocated at the first transfer that needs them.
+// them: the bytes of a small transfer, else one chunk of 8 MiB for each of its own up to CHUNKS,
+// allocated at the first transfer that needs them.
 struct Transfer {
     static constexpr int CHUNKS = 4;
     char* pin = nullptr;

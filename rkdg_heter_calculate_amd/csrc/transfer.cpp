@@ -21,10 +21,12 @@ namespace {
 
 constexpr size_t ONE_SHOT = (size_t)3 << 19;  // up to 1.5 MiB one copy and one memcpy are faster than threads
 constexpr size_t CHUNK = (size_t)8 << 20;     // 2 MiB chunks measured 2-3 times slower, larger ones no faster
+constexpr long long chunks_of(size_t n) { return (long long)((n + CHUNK - 1) / CHUNK); }
 
-// the pinned memory a transfer of n bytes wants; false: none to be had
-bool reserve(Transfer& t, size_t n) {
-    const size_t want = n <= ONE_SHOT ? ONE_SHOT : Transfer::CHUNKS * CHUNK;
+// the pinned memory a transfer of n bytes in nch chunks wants, no more than it can use (it is kept:
+// many small contexts hold little); false: none to be had
+bool reserve(Transfer& t, size_t n, long long nch) {
+    const size_t want = n <= ONE_SHOT ? (n + 4095) / 4096 * 4096 : (size_t)std::min<long long>(Transfer::CHUNKS, nch) * CHUNK;
     if (t.bytes >= want) return true;
     if (t.pin) (void)hipHostFree(t.pin);
     t.pin = nullptr;
@@ -86,7 +88,7 @@ struct Parts {
 int copy_ring(Transfer& t, hipStream_t s, const Parts& x) {
     const int B = Transfer::CHUNKS;
     const bool to_host = x.to_host;
-    const long long per = (long long)((x.n + CHUNK - 1) / CHUNK), nch = x.parts * per;  // chunks of a part, of all
+    const long long per = chunks_of(x.n), nch = x.parts * per;  // chunks of a part, of all
     auto chunk = [&](long long c, size_t& hoff, size_t& doff) {
         doff = (size_t)(c % per) * CHUNK;
         hoff = (size_t)(c / per) * x.n + doff;
@@ -168,7 +170,7 @@ int copy(Transfer& t, void* stream, const Parts& x) {
     hipStream_t s = (hipStream_t)stream;
     const size_t total = x.n * x.parts;
     char* pin = nullptr;
-    if (total > 0 && reserve(t, total)) {
+    if (total > 0 && reserve(t, total, x.parts * chunks_of(x.n))) {
         if (total > ONE_SHOT) {
             const int e = copy_ring(t, s, x);
             if (e >= 0) return e;
