@@ -217,18 +217,17 @@ int rkdg_batch_get_state(rkdg_batch* b, int32_t i, int32_t basis, double* U);
 int rkdg_batch_advance(rkdg_batch* b, int32_t nsteps, int32_t use_graph);
 int rkdg_batch_time(rkdg_batch* b, int32_t i, double* t);
 int rkdg_batch_sync(rkdg_batch* b);
-/* Autotuner: times every tile configuration the batch admits (rkdg_batch_set_tiles, and the
- * four-lanes-per-element tiles) on a repeatable stage and keeps the fastest; best_block may be
- * NULL. */
+/* Autotuner: times every tile configuration the batch admits (rkdg_batch_set_tiles) on a
+ * repeatable stage and keeps the fastest; best_block may be NULL. */
 int rkdg_batch_autotune(rkdg_batch* b, int32_t* best_block);
-/* Selects one tile configuration: staged != 0 for the staged 256-element tiles (FP64 form:
- * P1/P2; precision forms: P1-P3; when every tile's halo fits its LDS image), else
- * global-gather tiles of block = 64, 128 or 256 elements (the FP32-MFMA form: 64; the
- * BF16-MFMA form has staged tiles only); per_cu 0 launches one workgroup per tile, 4 or 8 a
- * persistent grid of that many 256-thread workgroups per CU.  RKDG_ERR_ARG when the batch
- * does not admit it.  rkdg_batch_get_tiles reports the configuration in use as
- * {staged, block, per_cu}; staged 2: the FP64 form's four-lanes-per-element tiles, which
- * rkdg_batch_create (with block 0) and the autotuner choose by themselves. */
+/* Selects one tile configuration: staged 2 with block 64 (P1, P2) or 128 (P3) and per_cu 0 for
+ * the FP64 form's four-lanes-per-element tiles (when every tile's edge lists fit), any other
+ * staged != 0 for the staged 256-element tiles (FP64 form: P1/P2; precision forms: P1-P3; when
+ * every tile's halo fits its LDS image), else global-gather tiles of block = 64, 128 or 256
+ * elements (the FP32-MFMA form: 64; the BF16-MFMA form has staged tiles only); per_cu 0 launches
+ * one workgroup per tile, 4 or 8 a persistent grid of that many 256-thread workgroups per CU.
+ * RKDG_ERR_ARG when the batch does not admit it.  rkdg_batch_get_tiles reports the configuration
+ * in use as {staged, block, per_cu}, which rkdg_batch_set_tiles takes back. */
 int rkdg_batch_set_tiles(rkdg_batch* b, int32_t staged, int32_t block, int32_t per_cu);
 int rkdg_batch_get_tiles(rkdg_batch* b, int32_t out[3]);
 int rkdg_batch_info(rkdg_batch* b, int64_t out[4]);   /* instances, total elements, block, device bytes */

@@ -594,7 +594,10 @@ static int device_cus(int dev) {
 // every halo fits the LDS image), or global-gather tiles of 64, 128 or 256 elements (the
 // precision form's global-gather kernel takes 64-element tiles only); per_cu 0 launches
 // one workgroup per tile, else a persistent grid of per_cu 256-thread workgroups per CU.
+// Staged 2 with their block: the four-lanes-per-element tiles, one workgroup per tile.
+static bool is_quad(const rkdg_batch* b, int staged, int block) { return staged == 2 && block == quad_block(b->P); }
 static bool tiles_valid(const rkdg_batch* b, int staged, int block, int per_cu) {
+    if (is_quad(b, staged, block)) return b->quad_ok && per_cu == 0;
     if (per_cu != 0 && per_cu != 4 && per_cu != 8) return false;
     if (staged) {
         if (b->prm.precision != RKDG_PREC_FP64) return b->staged_ok && block == px_block(b->P);
@@ -621,7 +624,7 @@ int rkdg_batch_set_tiles(rkdg_batch* b, int32_t staged, int32_t block, int32_t p
     if (!tiles_valid(b, staged, block, per_cu))
         return bfail(b, RKDG_ERR_ARG, "tile configuration not available for this batch");
     BCHK(b, hipSetDevice(b->dev));
-    return apply_tiles(b, staged ? 1 : 0, block, per_cu);
+    return apply_tiles(b, is_quad(b, staged, block) ? 2 : (staged ? 1 : 0), block, per_cu);
 }
 
 int rkdg_batch_get_tiles(rkdg_batch* b, int32_t out[3]) {
@@ -657,7 +660,7 @@ int rkdg_batch_autotune(rkdg_batch* b, int32_t* best_block) {
     for (int st = 0; st <= 2; ++st)
         for (int c : cands)
             for (int pw : pers) {
-                if (st < 2 ? !tiles_valid(b, st, c, pw) : !(b->quad_ok && c == quad_block(b->P) && pw == 0)) continue;
+                if (!(st < 2 || is_quad(b, st, c)) || !tiles_valid(b, st, c, pw)) continue;
                 int rc = apply_tiles(b, st, c, pw);
                 if (rc) return finish(rc, b->err);
                 // stage 1 reads buffers 1 and 0 and writes buffer 2: repeatable without

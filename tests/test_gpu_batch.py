@@ -95,7 +95,8 @@ def test_autotuned_batch_matches_oracle(P, prec):
     b.close()
 
 
-CONFIGS = [("fp64", 1, 256, pw) for pw in (0, 4, 8)] + \
+CONFIGS = [("fp64", 2, 64, 0)] + \
+          [("fp64", 1, 256, pw) for pw in (0, 4, 8)] + \
           [("fp64", 0, blk, pw) for blk in (64, 128, 256) for pw in (0, 4, 8)] + \
           [("fp32", 1, 256, pw) for pw in (0, 4, 8)] + [("fp32", 0, 64, pw) for pw in (0, 4, 8)] + \
           [("bf16", 1, 256, pw) for pw in (0, 4, 8)]

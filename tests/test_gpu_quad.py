@@ -152,8 +152,23 @@ def test_batch_instances_equal_single_meshes(P, flux):
         s.advance(5)
         assert np.array_equal(b.get_state(i, BASIS_NATIVE), s.get_state(BASIS_NATIVE)), i
         assert b.time(i) == s.time()[0]
-    with pytest.raises(Exception):  # chosen by the library, not through set_tiles
-        b.set_tiles(2, b.tiles()["block"], 0)
+    # the configuration reported can be given back, after another one
+    default = b.tiles()
+    b.set_tiles(0, 256, 8)
+    assert b.tiles() == {"staged": 0, "block": 256, "per_cu": 8}
+    b.set_tiles(**default)
+    assert b.tiles() == default
+    for i, s in enumerate(singles):
+        b.set_state(i, U := noisy_state(s, i), BASIS_NATIVE)
+        s.set_state(U, BASIS_NATIVE)
+        s.advance(2)
+    b.advance(2)
+    b.sync()
+    for i, s in enumerate(singles):
+        assert np.array_equal(b.get_state(i, BASIS_NATIVE), s.get_state(BASIS_NATIVE)), i
+    for block, per_cu in ((64 if P == 3 else 128, 0), (default["block"], 4)):
+        with pytest.raises(L.RkdgError):
+            b.set_tiles(2, block, per_cu)
     b.close()
 
 
