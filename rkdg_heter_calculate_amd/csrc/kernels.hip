@@ -1646,7 +1646,7 @@ __global__ void __launch_bounds__(256) k_fill_tables() {
     }
 }
 
-int upload_tables(int P, const DevTables& t) {
+static int fill_device_tables(int P, const DevTables& t) {
     hipError_t rc = hipMemcpyToSymbol(HIP_SYMBOL(c_tab), &t, sizeof(DevTables), (size_t)(P - 1) * sizeof(DevTables),
                                       hipMemcpyHostToDevice);
     if (rc != hipSuccess) return (int)rc;
@@ -1661,6 +1661,22 @@ int upload_tables(int P, const DevTables& t) {
     else hipLaunchKernelGGL(k_fill_tables<3>, dim3(1), dim3(256), 0, nullptr);
     rc = hipGetLastError();
     return (int)(rc == hipSuccess ? hipStreamSynchronize(nullptr) : rc);  // before any other stream reads them
+}
+
+// The tables depend on the degree alone: each device gets a degree's once, before the first context
+// that runs it, and kernels of other contexts never see them written.
+int upload_tables(int P, const DevTables& t) {
+    static std::mutex mu;
+    static bool there[NOALLOC_MAX_DEVICES][3] = {};
+    int dev = 0;
+    const hipError_t rc = hipGetDevice(&dev);
+    if (rc != hipSuccess) return (int)rc;
+    std::lock_guard<std::mutex> lk(mu);
+    if (dev >= NOALLOC_MAX_DEVICES) return fill_device_tables(P, t);
+    if (there[dev][P - 1]) return (int)hipSuccess;
+    const int e = fill_device_tables(P, t);
+    there[dev][P - 1] = e == (int)hipSuccess;
+    return e;
 }
 
 static int grid_blocks(const StageArgs& a) {
