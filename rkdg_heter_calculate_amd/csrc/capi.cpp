@@ -32,9 +32,9 @@ int host_threads() {
     return (int)std::min<unsigned>(hw ? hw : 1, 16);
 }
 
-void parallel_for(int n, const std::function<void(int, int)>& body) {
+void parallel_for(int n, const std::function<void(int, int)>& body, int few) {
     const int nt = host_threads();
-    if (n < 4096 || nt <= 1) { body(0, n); return; }
+    if (n < few || nt <= 1) { body(0, n); return; }
     std::vector<std::thread> th;
     int chunk = (n + nt - 1) / nt;
     for (int t = 0; t < nt; ++t) {
@@ -115,26 +115,32 @@ bool build_quad_lists(const int* nbr, long long ld, int E, int B, int hmax, std:
             }
         return (int)h.size() <= hmax;
     };
+    // first each tile's lists at their largest size, then packed to the capacities found
+    const int cap = 3 * B + hmax, few = 96;  // (a tile takes about 2 us, starting the threads 100)
+    std::vector<int> raw((size_t)ntiles * cap);
     std::atomic<bool> ok{true};
     parallel_for(ntiles, [&](int a, int b) {
         std::vector<int> jobs, h;
         for (int t = a; t < b && ok; ++t) {
-            if (!tile(t, jobs, h)) ok = false;
+            if (!tile(t, jobs, h)) {
+                ok = false;
+                break;
+            }
             nj[t] = (int)jobs.size();
             nh[t] = (int)h.size();
+            std::copy(h.begin(), h.end(), std::copy(jobs.begin(), jobs.end(), &raw[(size_t)t * cap]));
         }
-    });
+    }, few);
     if (!ok) return false;
     jcap = (*std::max_element(nj.begin(), nj.end()) + 15) / 16 * 16;
     hcap = (*std::max_element(nh.begin(), nh.end()) + 15) / 16 * 16;
     list.assign((size_t)ntiles * (jcap + hcap), -1);
     parallel_for(ntiles, [&](int a, int b) {
-        std::vector<int> jobs, h;
         for (int t = a; t < b; ++t) {
-            tile(t, jobs, h);
+            const int* r = &raw[(size_t)t * cap];
             int* l = &list[(size_t)t * (jcap + hcap)];
-            std::copy(jobs.begin(), jobs.end(), l);
-            std::copy(h.begin(), h.end(), l + jcap);
+            std::copy(r, r + nj[t], l);
+            std::copy(r + nj[t], r + nj[t] + nh[t], l + jcap);
         }
     });
     return true;

@@ -86,7 +86,8 @@ struct DevState {
 };
 
 // Minimal fork-join helper for host loops (the library carries no OpenMP runtime).
-void parallel_for(int n, const std::function<void(int, int)>& body);
+// Fewer than `few` iterations run on the caller's thread.
+void parallel_for(int n, const std::function<void(int, int)>& body, int few = 4096);
 int host_threads();  // its threads at most (RKDG_HOST_THREADS)
 
 // Pinned chunks for state transfers (transfer.cpp), kept with the context or batch that owns
