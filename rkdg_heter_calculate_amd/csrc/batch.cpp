@@ -378,7 +378,7 @@ int rkdg_batch_create(int32_t n, const rkdg_mesh* meshes, const rkdg_params* par
     BCREATECHK(hipMalloc(&b->rows, rows));
     b->bytes = sizeof(int) * (size_t)ld + rows + 3 * ub + sizeof(double) * hgeo.size() + sizeof(int) * hnbr.size() + hflag.size();
     const bool prec_form = p0.precision != RKDG_PREC_FP64;
-    if (!prec_form && env_int("RKDG_QUAD", 1)) {
+    if (!prec_form && quad_lds_bytes(b->P) <= max_lds_per_block(b->dev) && env_int("RKDG_QUAD", 1)) {
         std::vector<int> list;
         if (build_quad_lists(hnbr.data(), ld, (int)ld, quad_block(b->P), quad_halo(b->P), list, b->jcap, b->hcap)) {
             BCREATECHK(hipMalloc(&b->qlist, sizeof(int) * list.size()));

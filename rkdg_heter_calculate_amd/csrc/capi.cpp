@@ -378,7 +378,8 @@ int rkdg_create(const rkdg_mesh* m, const rkdg_params* prm, rkdg_ctx** out) {
     // smaller ones (P1, P2: 64 elements against 256), only up to the tiles that the
     // allocation-free step accepts: 4.2M elements, above which it would refuse the mesh.
     const bool noalloc_fits = c->block <= quad_block(c->P) || (c->E - 1) / quad_block(c->P) < NOALLOC_MAX_TILES;
-    const bool want_quad = prm->precision == RKDG_PREC_FP64 && prm->block == 0 && noalloc_fits && !std::getenv("RKDG_BLOCK") &&
+    const bool want_quad = prm->precision == RKDG_PREC_FP64 && prm->block == 0 && noalloc_fits &&
+                           quad_lds_bytes(c->P) <= max_lds_per_block(prm->device) && !std::getenv("RKDG_BLOCK") &&
                            !std::getenv("RKDG_STAGED") && !std::getenv("RKDG_PIPE") && !std::getenv("RKDG_PERSIST") &&
                            env_int("RKDG_QUAD", c->P == 3 || prm->flux == RKDG_FLUX_ROE || c->E <= quad_max_lf(c->P));
     c->xcd_remap = env_int("RKDG_XCD_REMAP", 1);

@@ -20,6 +20,7 @@
 // workgroup b runs on XCD b%8, and it processes tile (b%8)*(tiles/8) + b/8 so that each
 // XCD sweeps one contiguous range of elements and neighbour gathers hit its own L2.
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <climits>
 #include <mutex>
 #include <cstdlib>
@@ -1685,12 +1686,22 @@ static int grid_blocks(const StageArgs& a) {
     return nb;
 }
 
+// A kernel whose LDS exceeds 64 KiB must opt in, on every device it runs on (done: a bit for each
+// that has; a failure leaves the attribute unset, and the launch fails and reports it).
+template <typename K>
+static void lds_opt_in(K* kernel, size_t lds, std::atomic<unsigned long long>& done) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return;
+    const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+    if (done & bit) return;
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess) done |= bit;
+}
+
 template <int P, int FLUX>
 static void launch_stage_q(const StageArgs& a, hipStream_t s) {
     constexpr size_t lds = (size_t)quad_lds_bytes(P);
-    static bool opted = false;  // above 64 KiB the kernel must opt in
-    if (lds > 65536 && !opted)
-        opted = hipFuncSetAttribute((const void*)k_stage_q<P, FLUX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    static std::atomic<unsigned long long> opted{0};
+    if (lds > 65536) lds_opt_in(k_stage_q<P, FLUX>, lds, opted);
     hipLaunchKernelGGL((k_stage_q<P, FLUX>), dim3(grid_blocks(a)), dim3(Quad<P>::NT), lds, s, a);
 }
 
@@ -1703,11 +1714,10 @@ static void launch_stage_pf(int block, const StageArgs& a, hipStream_t s) {
     }
     if (a.staged) {
         constexpr size_t lds = (size_t)4 * Deg<P>::Np * staged_stride(P) * sizeof(double);
-        static bool opted = false;  // above 64 KiB the kernels must opt in
-        if (lds > 65536 && !opted) {
-            // (a failure leaves the attribute unset: the launch then fails and reports it)
-            opted = hipFuncSetAttribute((const void*)k_stage<P, FLUX, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
-                    hipFuncSetAttribute((const void*)k_stage_pipe<P <= 2 ? P : 2, FLUX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+        static std::atomic<unsigned long long> opted{0}, opted_pipe{0};
+        if (lds > 65536) {
+            lds_opt_in(k_stage<P, FLUX, true>, lds, opted);
+            lds_opt_in(k_stage_pipe<P <= 2 ? P : 2, FLUX>, lds, opted_pipe);
         }
         if (P == 1 && a.pipe == 2 && !a.tile_mesh)  // + the LDS copy of 4 geometry rows
             hipLaunchKernelGGL((k_stage_rp<1, FLUX>), grid, blk, lds + 4 * staged_block(1) * sizeof(double), s, a);
@@ -1734,10 +1744,8 @@ static void launch_stage_mx_p(int flux, const StageArgs& a, hipStream_t s) {
 template <int P, int FLUX, int CT>
 static void launch_stage_px_pf(const StageArgs& a, hipStream_t s) {
     constexpr size_t lds = (size_t)4 * Deg<P>::Np * staged_stride(P) * sizeof(double);
-    static bool opted = false;  // above 64 KiB the kernel must opt in
-    if (lds > 65536 && !opted) {
-        opted = hipFuncSetAttribute((const void*)k_stage_px<P, FLUX, CT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-    }
+    static std::atomic<unsigned long long> opted{0};
+    if (lds > 65536) lds_opt_in(k_stage_px<P, FLUX, CT>, lds, opted);
     hipLaunchKernelGGL((k_stage_px<P, FLUX, CT>), dim3(grid_blocks(a)), dim3(staged_block(P)), lds, s, a);
 }
 
@@ -1751,16 +1759,13 @@ template <int FLUX, int CT>
 static void launch_stage_pz_f(const StageArgs& a, hipStream_t s) {
     if (a.quad) {
         constexpr size_t lds = qf_lds(FLUX, CT);
-        static bool opted_q = false;  // above 64 KiB the kernel must opt in
-        if (lds > 65536 && !opted_q)
-            opted_q = hipFuncSetAttribute((const void*)k_stage_qf<FLUX, CT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+        static std::atomic<unsigned long long> opted_q{0};
+        if (lds > 65536) lds_opt_in(k_stage_qf<FLUX, CT>, lds, opted_q);
         hipLaunchKernelGGL((k_stage_qf<FLUX, CT>), dim3(grid_blocks(a)), dim3(Quad<3>::NT), lds, s, a);
         return;
     }
-    static bool opted = false;  // above 64 KiB the kernel must opt in
-    if (!opted) {
-        opted = hipFuncSetAttribute((const void*)k_stage_pz<3, FLUX, CT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Pz<3>::lds(CT)) == hipSuccess;
-    }
+    static std::atomic<unsigned long long> opted{0};
+    lds_opt_in(k_stage_pz<3, FLUX, CT>, Pz<3>::lds(CT), opted);
     hipLaunchKernelGGL((k_stage_pz<3, FLUX, CT>), dim3(grid_blocks(a)), dim3(Pz<3>::B), Pz<3>::lds(CT), s, a);
 }
 
