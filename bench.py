@@ -371,11 +371,11 @@ def main():
     per_launch = B * E
     avg_launch_ms = total_ms / (3 * args.steps)  # the stage kernels back to back, gaps included
     achieved = per_launch / (avg_launch_ms / 1e3) / 1e9
+    tiles = s.tiles()
     if lowp:
-        kfam = "k_stage_qf" if P == 3 else "k_stage_px"
-    else:  # four lanes per element at P3 and on the meshes that are small for the one-lane forms
-        small = E <= {1: 65536, 2: 640000, 3: E}[P]
-        kfam = "k_stage_q" if small else ("k_stage_rp" if P == 1 else "k_stage")
+        kfam = "k_stage_qf" if tiles["staged"] == 2 else ("k_stage_pz" if P == 3 else "k_stage_px")
+    else:  # four lanes per element, persistent staged tiles (P1 LF), or one tile per workgroup
+        kfam = "k_stage_q" if tiles["staged"] == 2 else ("k_stage_rp" if tiles["per_cu"] else "k_stage")
     kname = f"{kfam}_bf16_p{P}" if args.form == "bf16" else f"{kfam}_p{P}"
     traffic = read_traffic(f"{kname}_lf_{args.n}x{args.n}_hbm.md")
 

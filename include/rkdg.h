@@ -195,6 +195,9 @@ int rkdg_measure_copy(int32_t device, int64_t bytes, int32_t reps, double* gbs);
 
 /* Sizes the library derives: Np, Nqv, Nqe, n_elements, device bytes. */
 int rkdg_info(rkdg_ctx* ctx, int64_t out[5]);
+/* The tiles the context runs, as rkdg_batch_get_tiles: {staged, block, per_cu}; staged 2: the
+ * four-lanes-per-element tiles (FP64, and the P3 precision forms). */
+int rkdg_get_tiles(rkdg_ctx* ctx, int32_t out[3]);
 
 const char* rkdg_last_error(rkdg_ctx* ctx);   /* NULL ctx: last global error */
 const char* rkdg_strerror(int32_t code);

@@ -76,6 +76,7 @@ SIGNATURES = [
     ("rkdg_error_vs_exact", c_int32, [ctypes.c_void_p, c_int32, P_double, c_int32, P_double]),
     ("rkdg_measure_copy", c_int32, [c_int32, c_int64, c_int32, P_double]),
     ("rkdg_info", c_int32, [ctypes.c_void_p, P_int64]),
+    ("rkdg_get_tiles", c_int32, [ctypes.c_void_p, P_int32]),
     ("rkdg_last_error", ctypes.c_char_p, [ctypes.c_void_p]),
     ("rkdg_strerror", ctypes.c_char_p, [c_int32]),
     ("rkdg_step_noalloc", c_int32, [ctypes.c_void_p, c_double, ctypes.c_void_p, ctypes.c_void_p]),

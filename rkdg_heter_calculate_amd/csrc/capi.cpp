@@ -1135,6 +1135,16 @@ int rkdg_measure_copy(int32_t device, int64_t bytes, int32_t reps, double* gbs) 
     return RKDG_OK;
 }
 
+int rkdg_get_tiles(rkdg_ctx* c, int32_t out[3]) {
+    if (!c || !out) return fail(c, RKDG_ERR_ARG, "get_tiles");
+    int cus = 0;
+    HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->dev));
+    out[0] = c->quad ? 2 : c->staged;
+    out[1] = c->block;
+    out[2] = cus > 0 ? c->persistent / cus : 0;
+    return RKDG_OK;
+}
+
 int rkdg_info(rkdg_ctx* c, int64_t out[5]) {
     if (!c || !out) return RKDG_ERR_ARG;
     out[0] = c->Np; out[1] = c->Nqv; out[2] = c->Nqe; out[3] = c->E; out[4] = (int64_t)c->bytes;

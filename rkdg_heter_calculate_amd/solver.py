@@ -292,6 +292,11 @@ class Solver:
         self._chk(self.lib.rkdg_info(self.h, out.ctypes.data_as(L.P_int64)), "info")
         return {"Np": int(out[0]), "Nqv": int(out[1]), "Nqe": int(out[2]), "E": int(out[3]), "bytes": int(out[4])}
 
+    def tiles(self):
+        out = np.zeros(3, np.int32)
+        self._chk(self.lib.rkdg_get_tiles(self.h, L.iptr(out)), "get_tiles")
+        return {"staged": int(out[0]), "block": int(out[1]), "per_cu": int(out[2])}
+
 
 class Batch:
     """Many independent meshes advanced together, one launch per stage (rkdg_batch_*).

@@ -115,10 +115,12 @@ def test_every_tile_configuration_matches_oracle(prec, staged, block, per_cu):
     b.close()
 
 
-def test_farfield_instances_match_oracle():
+@pytest.mark.parametrize("tiles", [None, (1, 256, 0), (1, 256, 4), (0, 64, 0), (0, 256, 8)])
+def test_farfield_instances_match_oracle(tiles):
     """Far-field edges take the launch's free stream: two far-field meshes that share it,
-    beside a periodic mesh whose (unused) free-stream parameter differs."""
-    print("case: batch with far-field instances", flush=True)
+    beside a periodic mesh whose (unused) free-stream parameter differs; on the default
+    (four-lanes-per-element) tiles, the staged and the global-gather ones."""
+    print(f"case: batch with far-field instances, tiles {tiles}", flush=True)
     uinf, vinf = 0.5, 0.3
     fs = (1.0, uinf, vinf, 1.0 / 0.4 + 0.5 * (uinf * uinf + vinf * vinf))
     vp_open = [1.4, 3.0, uinf, vinf, 0.0, 0.0, 0.0, 0.0, 0.0]  # no periodic images
@@ -130,6 +132,9 @@ def test_farfield_instances_match_oracle():
     fss = [fs, (2.0, 0.0, 0.0, 9.0), fs]
     b = Batch([g for g, _, _ in inst], [dict(degree=2, dt_policy="max", cfl=c, freestream=list(f))
                                         for (_, _, c), f in zip(inst, fss)])
+    if tiles:
+        b.set_tiles(*tiles)
+    assert tuple(b.tiles().values()) == (tiles or (2, 64, 0))
     for i, (_, vp, _) in enumerate(inst):
         b.project_ic(i, 1, vp)
     b.advance(STEPS)

@@ -1,8 +1,9 @@
 """GPU against the oracle at the workloads' full sizes (the oracle takes seconds there).
 
 * the 512x512 jittered vortex mesh of the P2 benchmark (seed 2024, 524,288 triangles,
-  2,048 staged tiles, XCD-remapped sweep, halo capacity checked per tile), 5 steps, in
-  the FP64 form (1e-12) and the FP32-MFMA form (1e-6);
+  XCD-remapped sweep, halo capacity checked per tile), 5 steps, in the FP64 form (1e-12) on
+  8,192 four-lanes-per-element tiles and on the 2,048 staged tiles that larger meshes run, and
+  in the FP32-MFMA form (1e-6, staged tiles);
 * the 1024x1024 four-quadrant Riemann mesh (seed 2025, 2,097,152 triangles), P1, Roe,
   TVB M = 50 with positivity scaling, 3 steps (1e-12, equal limiter flags);
 * the same problem shrunk to 64x64 and run to t = 0.3 (about 3,500 steps), where the
@@ -39,12 +40,14 @@ def vortex_512_reference():
     return _REF["v512"]
 
 
-@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-6)])
-def test_vortex_p2_512_matches_oracle(prec, tol):
-    print(f"case: 512x512 P2 vortex 5 steps {prec}", flush=True)
+@pytest.mark.parametrize("prec,tol,quad", [("fp64", 1e-12, "1"), ("fp64", 1e-12, "0"), ("fp32", 1e-6, "0")])
+def test_vortex_p2_512_matches_oracle(prec, tol, quad, monkeypatch):
+    print(f"case: 512x512 P2 vortex 5 steps {prec} RKDG_QUAD={quad}", flush=True)
+    monkeypatch.setenv("RKDG_QUAD", quad)
     g, U0, Uo, to, M = vortex_512_reference()
     assert g.n_elements == 524288
     s = Solver(g, degree=2, flux="lf", dt_policy="max", cfl=0.3, precision=prec)
+    assert tuple(s.tiles().values()) == ((2, 64, 0) if quad == "1" else (1, 256, 0))
     s.set_state(U0)
     n, t = s.advance(5)
     # the time sums CFL dts of cell means: 1e-13 in FP64, the form's bar in FP32
@@ -70,13 +73,14 @@ def vortex_p3_1024_reference():
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-6), ("bf16", 2e-4)])
 def test_vortex_p3_1024_matches_oracle(prec, tol):
-    """P3 Roe on 2,097,152 triangles, 2 steps: the FP64 global-gather kernel (64-element
-    tiles) and the precision form's FP32-image tiles (256 elements, halo capacity checked per
-    tile) against the oracle."""
+    """P3 Roe on 2,097,152 triangles, 2 steps: the four-lanes-per-element tiles of the FP64 form
+    and of the precision forms (128 elements, halo capacity checked per tile) against the
+    oracle."""
     print(f"case: 1024x1024 P3 Roe vortex 2 steps {prec}", flush=True)
     g, kw, U0, Uo, to, M = vortex_p3_1024_reference()
     assert g.n_elements == 2097152
     s = Solver(g, precision=prec, **kw)
+    assert tuple(s.tiles().values()) == (2, 128, 0)
     s.set_state(U0)
     n, t = s.advance(2)
     assert n == 2 and abs(t - to) <= (1e-13 if prec == "fp64" else tol) * to

@@ -145,7 +145,7 @@ def test_run_twice_bitwise():
     assert np.array_equal(a, b)
 
 
-@pytest.mark.parametrize("P", [2, 1])  # P1 LF runs the register-pipelined persistent tiles
+@pytest.mark.parametrize("P", [2, 1])  # (the other FP64 forms: test_gpu_forms.py)
 def test_advance_counts_steps_per_call(P):
     print(f"case: advance step counts and end time P{P}", flush=True)
     g = vortex_grid(16, jitter=0.2, diagonal=1, seed=5)
@@ -164,7 +164,7 @@ def test_advance_counts_steps_per_call(P):
 
 
 def test_p1_pipelined_tiles_match_oracle(monkeypatch):
-    """P1 LF FP64 runs the register-pipelined persistent tile (next tile's image loaded into
+    """P1 LF FP64 above 65,536 elements runs the register-pipelined persistent tile (next tile's image loaded into
     registers during the current tile). 528 full tiles and a partial one on 256 workgroups
     (RKDG_PERSIST=1 on a 256-CU part) give each workgroup two or three tiles, so the
     prefetch chain (data one tile ahead, halo ids two, halo offsets three) runs; the result
@@ -389,8 +389,9 @@ def test_precision_form_vortex_steps():
 
 @pytest.mark.parametrize("P,flux", [(2, "roe"), (3, "lf"), (3, "roe")])
 def test_precision_form_staged_tiles_with_halos(P, flux):
-    """The lane-per-element precision kernels on a mesh of several 256-element tiles (halos
-    gathered from other tiles, padded lanes in the last tile): 10 steps against the oracle."""
+    """The precision kernels (P2: lane per element on 256-element tiles; P3: four lanes per element
+    on 128-element tiles) on a mesh of several tiles (halos gathered from other tiles, padded
+    lanes in the last tile): 10 steps against the oracle."""
     print(f"case: FP32-MFMA staged tiles P{P} {flux}", flush=True)
     g = vortex_grid(20, jitter=0.2, diagonal=1, seed=13)  # 800 triangles: 4 tiles, the last one partial
     o, _ = make_pair(g, P=P, flux=flux, dt_policy="max", cfl=0.2)
@@ -404,8 +405,9 @@ def test_precision_form_staged_tiles_with_halos(P, flux):
     assert np.all(err < MX_TOL), err
     assert np.all(err > 0)
     assert np.allclose(s.residual(), o.residual_change(), rtol=1e-3, atol=1e-15)
-    # the four-lanes-per-element kernel (RKDG_PX=0) rounds differently: a different result
-    # shows that the staged lane-per-element kernel ran
+    assert tuple(s.tiles().values()) == ((2, 128, 0) if P == 3 else (1, 256, 0))
+    # the 64-element form (RKDG_PX=0) rounds differently: a different result shows that the
+    # tiles' kernel ran
     import os
     os.environ["RKDG_PX"] = "0"
     try:
