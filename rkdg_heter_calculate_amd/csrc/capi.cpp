@@ -36,12 +36,14 @@ void parallel_for(int n, const std::function<void(int, int)>& body, int few) {
     const int nt = host_threads();
     if (n < few || nt <= 1) { body(0, n); return; }
     std::vector<std::thread> th;
-    int chunk = (n + nt - 1) / nt;
-    for (int t = 0; t < nt; ++t) {
-        int a = t * chunk, b = std::min(n, a + chunk);
-        if (a >= b) break;
-        th.emplace_back(body, a, b);
+    const int chunk = (n + nt - 1) / nt;
+    int a = 0;  // iterations handed out
+    try {
+        th.reserve(nt);
+        for (; a < n; a += chunk) th.emplace_back(std::cref(body), a, std::min(n, a + chunk));
+    } catch (...) {  // no (more) threads to be had: the rest runs here
     }
+    if (a < n) body(a, n);
     for (auto& x : th) x.join();
 }
 
@@ -87,49 +89,46 @@ int build_halo(const int* nbr, long long ld, int E, int B, std::vector<int>& hof
 bool build_quad_lists(const int* nbr, long long ld, int E, int B, int hmax, std::vector<int>& list, int& jcap, int& hcap) {
     const int ntiles = (E + B - 1) / B;
     std::vector<int> nj(ntiles, 0), nh(ntiles, 0);
-    // one tile's edges and halo entries; false: an edge that is not paired with the edge that
-    // points back (or with itself), which only a form that computes both sides can run
-    auto tile = [&](int t, std::vector<int>& jobs, std::vector<int>& h) {
+    // one tile's edges, its halo entries behind them; returns the latter's number, or -1: too many, or
+    // an edge that is not paired with the edge that points back (or with itself), which only a form
+    // that computes both sides can run
+    constexpr int MAXB = 128;
+    if (B > MAXB) return false;
+    auto tile = [&](int t, int* jobs, int& njobs) {  // (workers allocate nothing)
         const int lo = t * B, hi = std::min(E, lo + B);
-        jobs.clear();
-        h.clear();
+        int h[3 * MAXB], nhalo = 0;
+        njobs = 0;
         for (int k = 0; k < 3; ++k)
             for (int p = lo; p < hi; ++p) {
                 const int w = nbr[(size_t)k * ld + p];
-                if (w >= 0 && ((w >> 2) < lo || (w >> 2) >= hi)) h.push_back(w);
+                if (w >= 0 && ((w >> 2) < lo || (w >> 2) >= hi)) h[nhalo++] = w;
             }
-        std::sort(h.begin(), h.end());
+        if (nhalo > hmax) return -1;
+        std::sort(h, h + nhalo);
         for (int k = 0; k < 3; ++k)
             for (int p = lo; p < hi; ++p) {
                 const int w = nbr[(size_t)k * ld + p], row = k * B + p - lo, n = w >> 2;
                 int far = w;  // -tag
                 if (w >= 0 && n >= lo && n < hi) {
-                    if (nbr[(size_t)(w & 3) * ld + n] != ((p << 2) | k)) return false;
+                    if (nbr[(size_t)(w & 3) * ld + n] != ((p << 2) | k)) return -1;
                     far = (w & 3) * B + n - lo;
-                    if (far == row) return false;
+                    if (far == row) return -1;
                     if (far < row) continue;  // listed from the other side
                 } else if (w >= 0) {
-                    far = 3 * B + (int)(std::lower_bound(h.begin(), h.end(), w) - h.begin());
+                    far = 3 * B + (int)(std::lower_bound(h, h + nhalo, w) - h);
                 }
-                jobs.push_back(row | (far + 8) << 9);
+                jobs[njobs++] = row | (far + 8) << 9;
             }
-        return (int)h.size() <= hmax;
+        std::copy(h, h + nhalo, jobs + njobs);
+        return nhalo;
     };
     // first each tile's lists at their largest size, then packed to the capacities found
     const int cap = 3 * B + hmax, few = 96;  // (a tile takes about 2 us, starting the threads 100)
     std::vector<int> raw((size_t)ntiles * cap);
     std::atomic<bool> ok{true};
     parallel_for(ntiles, [&](int a, int b) {
-        std::vector<int> jobs, h;
-        for (int t = a; t < b && ok; ++t) {
-            if (!tile(t, jobs, h)) {
-                ok = false;
-                break;
-            }
-            nj[t] = (int)jobs.size();
-            nh[t] = (int)h.size();
-            std::copy(h.begin(), h.end(), std::copy(jobs.begin(), jobs.end(), &raw[(size_t)t * cap]));
-        }
+        for (int t = a; t < b && ok; ++t)
+            if ((nh[t] = tile(t, &raw[(size_t)t * cap], nj[t])) < 0) ok = false;
     }, few);
     if (!ok) return false;
     jcap = (*std::max_element(nj.begin(), nj.end()) + 15) / 16 * 16;

@@ -463,3 +463,31 @@ def test_mesh_writer_round_trip_naca(tmp_path):
     r = Grid.read(str(out / "mesh.conf"), str(out / "ElemDepart.dat"), box=15.0)
     _assert_same_mesh(g, r)
     assert np.array_equal(r.partition, g.partition)
+
+
+def test_host_loops_without_threads(tmp_path):
+    """Where no thread can be started (no address space for its stack) the host loops run on the
+    caller's thread: the same values, and no exception out of the C entry."""
+    import subprocess
+    import sys
+    prog = tmp_path / "no_threads.py"
+    prog.write_text("""
+import resource, sys
+import numpy as np
+from rkdg_heter_calculate_amd import Grid, _lib as L
+g = Grid.splitquad(80, 80, 0.0, 0.0, 1.0, 1.0, periodic=False, diagonal=1, jitter=0.2, seed=1)
+ex, ey = (np.ascontiguousarray(a) for a in g.element_coords())
+U = np.random.default_rng(0).uniform(-1, 1, (4, 6, g.n_elements))
+a, b = np.empty_like(U), np.empty_like(U)
+conv = lambda out: L.load().rkdg_convert_basis(2, g.n_elements, L.dptr(ex), L.dptr(ey), 1, L.dptr(U), L.dptr(out))
+with open("/proc/self/statm") as f:
+    used = int(f.read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (1 << 20), resource.RLIM_INFINITY))
+rc = conv(a)
+resource.setrlimit(resource.RLIMIT_AS, (resource.RLIM_INFINITY, resource.RLIM_INFINITY))
+assert rc == 0 and conv(b) == 0 and np.array_equal(a, b)
+print("same")
+""")
+    env = dict(os.environ, RKDG_HOST_THREADS="8", PYTHONPATH=ROOT)
+    r = subprocess.run([sys.executable, str(prog)], capture_output=True, text=True, timeout=120, env=env)
+    assert r.returncode == 0 and r.stdout.strip() == "same", (r.returncode, r.stdout, r.stderr[-1000:])
