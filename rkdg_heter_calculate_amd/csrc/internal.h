@@ -268,8 +268,10 @@ constexpr int quad_ops(int P) {
 // Meshes of at most this many elements run it with LF at P1 and P2 too: the one-lane forms put
 // 256 elements on a workgroup and need one tile per CU at P1 (65,536 elements; P1 LF at 32,768 /
 // 65,522 / 125,000 triangles: 9.4 / 13.3 / 20.4 us per stage against 13.0 / 14.2 / 16.9) and
-// several at P2 (P2 LF at 20,000 / 262,088 / 524,288 / 2.1M: 10.7 / 42.2 / 81 / 322 against
-// 16.5 / 45.9 / 86.6 / 308; at 125,000, one exact round of their workgroups, 25.1 against 24.3).
+// several at P2 (P2 LF, 200 steps, this form against the staged tiles: 20,000 10.6 / 16.4; 125,000,
+// one exact round of their workgroups, 24.2 / 24.8; 262,088 41.4 / 47.0; 524,288 79.4 / 85.3;
+// 819,200 129 / 134; 1.05M 166 / 168; 1.41M 221 / 218; 2.1M 316 / 306: the line lies below the
+// crossing, where it was drawn from 524,288 and 2.1M alone).
 constexpr int quad_max_lf(int P) { return P == 1 ? 1 << 16 : (P == 2 ? 640000 : 0); }
 // Tile-boundary edges at most (Z-order tiles of 64 have 24-60, of 128 32-76): each of the tile's
 // lanes of a group takes at most one, so never more than the tile's elements.

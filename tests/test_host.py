@@ -465,6 +465,7 @@ def test_mesh_writer_round_trip_naca(tmp_path):
     assert np.array_equal(r.partition, g.partition)
 
 
+@pytest.mark.skipif("libasan" in os.environ.get("LD_PRELOAD", ""), reason="the sanitizer maps its own shadow memory")
 def test_host_loops_without_threads(tmp_path):
     """Where no thread can be started (no address space for its stack) the host loops run on the
     caller's thread: the same values, and no exception out of the C entry."""
