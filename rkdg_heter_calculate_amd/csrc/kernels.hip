@@ -1261,9 +1261,9 @@ __global__ void k_state_init(DevState* st, int n, int slot, double t) {
 // of theirs is fetching instructions no other wave has run in the launch (clock stamps at 131,072
 // triangles, P1: 11,500 cycles in the first half and 6,000 in the second, 3,200 where other waves
 // had been through it).  So the first half is one copy of its code for the four components (their
-// modes and means take turns in row 0): 32,768 triangles, four-quadrant problem, P1 11.9 -> 10.8 us
-// per launch, P2 14.2 -> 13.2; where every element is limited 9.3 -> 8.2 and 10.3 -> 9.2; and a.warm
-// sends every third workgroup of an XCD through the second half (launch_limiter).
+// modes and means take turns in row 0): 65,522 triangles, four-quadrant problem, P1 12.3 -> 11.3 us
+// per launch, P2 15.6 -> 15.0; where every element is limited 10.4 -> 9.4 and 12.5 -> 11.8; and
+// a.warm sends every third workgroup of an XCD through the second half (launch_limiter).
 constexpr double POS_EPS = 1e-13;
 
 template <int P>
